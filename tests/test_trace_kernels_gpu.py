@@ -1,0 +1,76 @@
+"""Kernels of the trace solve at the sizes where their tiling can go wrong.
+
+* the block-Jacobi inverse (several blocks per wavefront) against numpy's
+  inverse of the assembled diagonal blocks, for every block size of the 2-D
+  and 3-D orders and block counts that do not fill the last wavefront;
+* the reconstruction u = U lambda + U0, q = Q lambda + Q0 against numpy on the
+  same condensed blocks, for odd and even row lengths.
+
+Bounds: an inverse by Gauss-Jordan with partial pivoting is off by at most a
+few n eps cond(D) (n <= 21, cond(D) computed), a dot product of NL + 1 terms by
+(NL + 1) eps times the sum of the terms' magnitudes."""
+import numpy as np
+import pytest
+
+import hyperfox_amd as hf
+import hyperfox_amd.problems as pr
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(np.float64).eps
+
+
+def problem(dim, p, n):
+    w = pr.diffusion_source_2d(n, p) if dim == 2 else pr.convection_diffusion_3d(n, p)
+    prob = hf.HDGProblem(dim, p)
+    pr.setup_gpu(w, prob)
+    prob.assemble()
+    return w, prob
+
+
+def diagonal_blocks(w, prob):
+    bs = prob.sizes['nNf']
+    rowptr, cols, vals, _ = prob.trace_csr()
+    nb = w.mesh.n_faces
+    D = np.zeros((nb, bs, bs))
+    for F in range(nb):
+        for r in range(bs):
+            k0, k1 = rowptr[F * bs + r], rowptr[F * bs + r + 1]
+            k = k0 + int(np.where(cols[k0:k1] == F * bs)[0][0])
+            D[F, r] = vals[k:k + bs]
+    return D
+
+
+@pytest.mark.parametrize('dim,p,n', [(2, 1, 3), (2, 2, 2), (2, 3, 5), (2, 4, 3), (2, 5, 2), (2, 6, 1), (2, 7, 2),
+                                     (2, 8, 1), (2, 9, 2), (2, 10, 1), (3, 1, 2), (3, 2, 1), (3, 3, 2), (3, 4, 1),
+                                     (3, 5, 1)])
+def test_block_jacobi_inverse(dim, p, n):
+    print('block jacobi', dim, p, n, flush=True)
+    w, prob = problem(dim, p, n)
+    D = diagonal_blocks(w, prob)
+    bs = D.shape[1]
+    rng = np.random.default_rng(p)
+    x = rng.standard_normal((w.mesh.n_faces, bs))
+    y = prob.pc_apply(hf.PC_BJACOBI, x.reshape(-1)).reshape(-1, bs)
+    inv = np.linalg.inv(D)
+    ref = np.einsum('fij,fj->fi', inv, x)
+    cond = np.linalg.cond(D)
+    bound = 16 * bs * EPS * cond * np.linalg.norm(inv, axis=(1, 2)) * np.linalg.norm(x, axis=1)
+    assert (np.linalg.norm(y - ref, axis=1) <= bound).all()
+
+
+@pytest.mark.parametrize('dim,p,n', [(2, 1, 1), (2, 2, 3), (2, 3, 2), (2, 4, 3), (2, 5, 1), (2, 8, 1), (3, 1, 1),
+                                     (3, 2, 1), (3, 3, 1), (3, 4, 1), (3, 5, 1)])
+def test_reconstruction(dim, p, n):
+    print('reconstruct', dim, p, n, flush=True)
+    w, prob = problem(dim, p, n)
+    prob.set_krylov(hf.KRYLOV_BICGSTAB)
+    prob.solve(pc=hf.PC_BJACOBI, rtol=1e-8, maxits=5000)
+    u, q, lam = prob.solution()
+    c = prob.condensed()
+    a = w.mesh.arrays()
+    nNf = prob.sizes['nNf']
+    lc = lam.reshape(-1, nNf)[a['cell2face'][:, :, None], a['face_perm'].astype(int)].reshape(w.mesh.n_cells, -1)
+    for got, M, M0 in ((u, c['U'], c['U0']), (q, c['Q'], c['Q0'])):
+        ref = np.einsum('eij,ej->ei', M, lc) + M0
+        mag = np.einsum('eij,ej->ei', np.abs(M), np.abs(lc)) + np.abs(M0)
+        assert (np.abs(got - ref) <= 2 * (lc.shape[1] + 1) * EPS * mag).all()
