@@ -539,25 +539,29 @@ extern "C" int hfx_hdg_get_trace_csr(hfx_hdg* h, long long* rowptr, int* cols, d
 
 namespace {
 
-// Set up preconditioner `pc` on the assembled trace matrix; returns its apply
-// (empty for none).
-std::function<void(const double*, double*)> make_pc(hfx_hdg* h, int pc) {
+// Set up preconditioner `pc` on the assembled trace matrix.
+hfx::PcApply make_pc(hfx_hdg* h, int pc) {
   const long long n = h->A.nrows();
   hipStream_t s = h->stream;
-  std::function<void(const double*, double*)> M;
+  hfx::PcApply M;
   const auto t0 = std::chrono::steady_clock::now();
   if (pc == HFX_PC_JACOBI) {
     h->dinv.alloc(n);
     hfx::bsr_inv_point_diag(h->A, h->dinv.p, s);
-    M = [h, n, s](const double* in, double* out) { hfx::apply_point_diag(n, h->dinv.p, in, out, s); };
+    M.kind = hfx::PC_JACOBI;
+    M.dinv = h->dinv.p;
+    M.fn = [h, n, s](const double* in, double* out) { hfx::apply_point_diag(n, h->dinv.p, in, out, s); };
   } else if (pc == HFX_PC_BJACOBI) {
     h->dinv.alloc((size_t)h->A.nb * h->A.bs * h->A.bs);
     hfx::bsr_invert_diag(h->A, h->dinv.p, s);
-    M = [h, s](const double* in, double* out) { hfx::apply_block_diag(h->A.nb, h->A.bs, h->dinv.p, in, out, s); };
+    M.kind = hfx::PC_BJACOBI;
+    M.dinv = h->dinv.p;
+    M.fn = [h, s](const double* in, double* out) { hfx::apply_block_diag(h->A.nb, h->A.bs, h->dinv.p, in, out, s); };
   } else if (pc == HFX_PC_LEARNED) {
     hfx::lpc_prepare(h);
     const hfx::LpcInfer* st = h->lpc_state.get();
-    M = [st, s](const double* in, double* out) { hfx::bsr_spmv_f32vals(st->g, st->mvals.p, in, out, s); };
+    M.kind = hfx::PC_OTHER;
+    M.fn = [st, s](const double* in, double* out) { hfx::bsr_spmv_f32vals(st->g, st->mvals.p, in, out, s); };
   } else if (pc == HFX_PC_ILU0 || pc == HFX_PC_ILU0_NATURAL || pc == HFX_PC_ILU0_F32) {
     const int ord = pc == HFX_PC_ILU0_NATURAL ? hfx::ILU_NATURAL : hfx::ILU_MULTICOLOUR;
     if (!h->ilu || h->ilu->ordering != ord) {
@@ -567,7 +571,8 @@ std::function<void(const double*, double*)> make_pc(hfx_hdg* h, int pc) {
     h->ilu->low = pc == HFX_PC_ILU0_F32;
     h->ilu->factor(h->A, s);
     hfx::Ilu* f = h->ilu.get();
-    M = [f, s](const double* in, double* out) { f->apply(in, out, s); };
+    M.kind = hfx::PC_OTHER;
+    M.fn = [f, s](const double* in, double* out) { f->apply(in, out, s); };
   } else if (pc != HFX_PC_NONE) {
     throw std::runtime_error("hfx_hdg_solve: unknown preconditioner");
   }
@@ -599,14 +604,14 @@ void do_solve(hfx_hdg* h, int pc, double rtol, int maxits, int restart, hfx::Kry
     info.reason = hfx::CONVERGED_RTOL;
     return;
   }
-  std::function<void(const double*, double*)> M = make_pc(h, pc);
+  const hfx::PcApply M = make_pc(h, pc);
   HFX_HIP(hipMemsetAsync(h->lambda.p, 0, n * sizeof(double), s));
   hfx::KrylovOpts o;
   o.rtol = rtol;
   o.maxits = maxits;
   o.restart = restart;
   o.graph = h->solver_graphs;
-  if (h->krylov == HFX_KRYLOV_BICGSTAB) hfx::bicgstab(h->A, h->rhs.p, h->lambda.p, M, o, info, s);
+  if (h->krylov == HFX_KRYLOV_BICGSTAB) hfx::bicgstab(h->A, h->rhs.p, h->lambda.p, M, o, info, s, &h->kws);
   else hfx::fgmres(h->A, h->rhs.p, h->lambda.p, M, o, info, s);
 }
 
@@ -933,11 +938,11 @@ extern "C" int hfx_hdg_pc_apply(hfx_hdg* h, int pc, const double* x, double* y) 
   h->set_device();
   const long long n = h->A.nrows();
   hipStream_t s = h->stream;
-  std::function<void(const double*, double*)> M = make_pc(h, pc);
+  const hfx::PcApply M = make_pc(h, pc);
   hfx::DevBuf<double> dx, dy;
   dx.upload(x, n, s);
   dy.alloc(n);
-  if (M) M(dx.p, dy.p);
+  if (M.kind != hfx::PC_NONE) M.fn(dx.p, dy.p);
   else HFX_HIP(hipMemcpyAsync(dy.p, dx.p, n * sizeof(double), hipMemcpyDeviceToDevice, s));
   dy.download(y, n, s);
   HFX_HIP(hipStreamSynchronize(s));

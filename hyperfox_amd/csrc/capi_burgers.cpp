@@ -61,6 +61,7 @@ struct hfx_burgers {
   hfx::BsrPattern pat;
   hfx::BsrDev A;
   std::unique_ptr<hfx::Ilu> ilu;
+  hfx::KrylovWs kws;        // solver workspace
   void set_device() const { HFX_HIP(hipSetDevice(device)); }
   int bs() const { return mesh.nNf * m; }
   long long n_trace() const { return (long long)mesh.nFaces * bs(); }
@@ -169,19 +170,26 @@ void assemble(hfx_burgers* h) {
   h->assembled = true;
 }
 
-std::function<void(const double*, double*)> make_pc(hfx_burgers* h, int pc) {
+hfx::PcApply make_pc(hfx_burgers* h, int pc) {
   const long long n = h->A.nrows();
   hipStream_t s = h->stream;
-  if (pc == HFX_PC_NONE) return {};
+  hfx::PcApply M;
+  if (pc == HFX_PC_NONE) return M;
   if (pc == HFX_PC_JACOBI) {
     h->dinv.alloc(n);
     hfx::bsr_inv_point_diag(h->A, h->dinv.p, s);
-    return [h, n, s](const double* in, double* out) { hfx::apply_point_diag(n, h->dinv.p, in, out, s); };
+    M.kind = hfx::PC_JACOBI;
+    M.dinv = h->dinv.p;
+    M.fn = [h, n, s](const double* in, double* out) { hfx::apply_point_diag(n, h->dinv.p, in, out, s); };
+    return M;
   }
   if (pc == HFX_PC_BJACOBI) {
     h->dinv.alloc((size_t)h->A.nb * h->A.bs * h->A.bs);
     hfx::bsr_invert_diag(h->A, h->dinv.p, s);
-    return [h, s](const double* in, double* out) { hfx::apply_block_diag(h->A.nb, h->A.bs, h->dinv.p, in, out, s); };
+    M.kind = hfx::PC_BJACOBI;
+    M.dinv = h->dinv.p;
+    M.fn = [h, s](const double* in, double* out) { hfx::apply_block_diag(h->A.nb, h->A.bs, h->dinv.p, in, out, s); };
+    return M;
   }
   if (pc == HFX_PC_ILU0 || pc == HFX_PC_ILU0_F32) {
     if (!h->ilu) {  // kept only once its set-up succeeded
@@ -192,7 +200,9 @@ std::function<void(const double*, double*)> make_pc(hfx_burgers* h, int pc) {
     h->ilu->low = pc == HFX_PC_ILU0_F32;
     h->ilu->factor(h->A, s);
     hfx::Ilu* f = h->ilu.get();
-    return [f, s](const double* in, double* out) { f->apply(in, out, s); };
+    M.kind = hfx::PC_OTHER;
+    M.fn = [f, s](const double* in, double* out) { f->apply(in, out, s); };
+    return M;
   }
   throw std::runtime_error("hfx_burgers_solve: unsupported preconditioner");
 }
@@ -208,7 +218,7 @@ void solve(hfx_burgers* h, int pc, double rtol, int maxits, int restart, hfx::Kr
   o.maxits = maxits;
   o.restart = restart;
   o.graph = h->graphs;
-  if (h->krylov == HFX_KRYLOV_BICGSTAB) hfx::bicgstab(h->A, h->rhs.p, h->trace.p, M, o, info, s);
+  if (h->krylov == HFX_KRYLOV_BICGSTAB) hfx::bicgstab(h->A, h->rhs.p, h->trace.p, M, o, info, s, &h->kws);
   else hfx::fgmres(h->A, h->rhs.p, h->trace.p, M, o, info, s);
   const int mu = m.nN * h->m;
   hfx::launch_reconstruct(m.nCells, mu, mu * h->dim, m.nFpc, h->bs(), h->U.p, h->U0.p, h->Q.p, h->Q0.p, h->c2f.p,

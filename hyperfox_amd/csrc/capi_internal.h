@@ -106,6 +106,7 @@ struct hfx_hdg {
   double last_pc_setup_ms = 0.0;
   std::unique_ptr<hfx::Ilu> ilu;  // ILU(0) schedule + factors for the current pattern
   int krylov = HFX_KRYLOV_FGMRES;
+  hfx::KrylovWs kws;  // solver workspace
   bool solver_graphs = false;  // hfx_hdg_set_solver_graphs
   // last solve options
   int last_pc = HFX_PC_BJACOBI, last_maxits = 10000, last_restart = 30;

@@ -63,6 +63,7 @@ struct hfx_la {
   // device copy (uploaded by the first solve after a change)
   hfx::BsrDev A;
   hfx::DevBuf<double> db, dx, dinv;
+  hfx::KrylovWs kws;  // solver workspace
   bool dev_dirty = true;
   std::unique_ptr<hfx::Ilu> ilu;  // point ILU(0) of the uploaded matrix
   bool ilu_stale = true;
@@ -342,11 +343,13 @@ extern "C" int hfx_la_solve(hfx_la* h, double* x, int n, int* info, double* relr
     h->upload();
     hipStream_t s = h->stream;
     HFX_HIP(hipMemsetAsync(h->dx.p, 0, (size_t)h->n * sizeof(double), s));
-    std::function<void(const double*, double*)> M;
+    hfx::PcApply M;
     if (h->pc == HFX_PC_JACOBI) {
       const double* dinv = h->dinv.p;
       const long long nn = h->n;
-      M = [dinv, nn, s](const double* in, double* out) { hfx::apply_point_diag(nn, dinv, in, out, s); };
+      M.kind = hfx::PC_JACOBI;
+      M.dinv = dinv;
+      M.fn = [dinv, nn, s](const double* in, double* out) { hfx::apply_point_diag(nn, dinv, in, out, s); };
     } else if (h->pc == HFX_PC_ILU0 || h->pc == HFX_PC_ILU0_NATURAL) {
       const int ord = h->pc == HFX_PC_ILU0 ? hfx::ILU_MULTICOLOUR : hfx::ILU_NATURAL;
       if (h->ilu_stale || !h->ilu || h->ilu->ordering != ord) {
@@ -361,13 +364,14 @@ extern "C" int hfx_la_solve(hfx_la* h, double* x, int n, int* info, double* relr
         h->ilu_stale = false;
       }
       hfx::Ilu* f = h->ilu.get();
-      M = [f, s](const double* in, double* out) { f->apply(in, out, s); };
+      M.kind = hfx::PC_OTHER;
+      M.fn = [f, s](const double* in, double* out) { f->apply(in, out, s); };
     }
     hfx::KrylovOpts o;
     o.rtol = h->rtol;
     o.maxits = h->maxits;
     o.restart = h->restart;
-    if (h->solver == HFX_LA_BCGS) hfx::bicgstab(h->A, h->db.p, h->dx.p, M, o, ki, s);
+    if (h->solver == HFX_LA_BCGS) hfx::bicgstab(h->A, h->db.p, h->dx.p, M, o, ki, s, &h->kws);
     else hfx::fgmres(h->A, h->db.p, h->dx.p, M, o, ki, s);
     h->dx.download(x, h->n, s);
     HFX_HIP(hipStreamSynchronize(s));

@@ -15,7 +15,41 @@
 
 namespace hfx {
 
-enum PcType { PC_NONE = 0, PC_JACOBI = 1, PC_BJACOBI = 2, PC_LEARNED = 3 };
+enum PcType { PC_NONE = 0, PC_JACOBI = 1, PC_BJACOBI = 2, PC_OTHER = 3 };
+
+// A preconditioner set up on the matrix: fn(in, out) applies it (empty for
+// PC_NONE).  The solvers fuse point and block Jacobi into the vector kernel
+// before them and read dinv themselves.
+struct PcApply {
+  PcType kind = PC_NONE;
+  const double* dinv = nullptr;  // PC_JACOBI: n values, PC_BJACOBI: bs x bs row-major blocks
+  std::function<void(const double*, double*)> fn;
+};
+
+// What the device reports to the host while a solve runs (pinned memory).
+struct KrylovStatus {
+  int seq, code;
+};
+
+// Solver workspace of one problem handle, kept between solves: the vectors of
+// systems up to KEEP bytes (larger ones are allocated per solve, where the
+// allocation is lost in the solve) and the pinned status word.
+struct KrylovWs {
+  static constexpr size_t KEEP = (size_t)64 << 20;
+  DevBuf<double> mem;
+  KrylovStatus* status = nullptr;
+  KrylovWs() = default;
+  KrylovWs(const KrylovWs&) = delete;
+  KrylovWs& operator=(const KrylovWs&) = delete;
+  ~KrylovWs();
+  KrylovStatus* host();                     // allocated at first use, reset
+  void wait(int seq, hipStream_t s) const;  // until status->seq >= seq
+  double* mem_for(size_t doubles, DevBuf<double>& own) {
+    DevBuf<double>& m = doubles * sizeof(double) <= KEEP ? mem : own;
+    if (m.n < doubles) m.alloc(doubles);
+    return m.p;
+  }
+};
 
 // KSP converged reasons (a subset of PETSc's codes).
 enum SolveReason { CONVERGED_RTOL = 2, CONVERGED_ATOL = 3, DIVERGED_ITS = -3, DIVERGED_BREAKDOWN = -5, DIVERGED_NANORINF = -9 };
@@ -69,22 +103,22 @@ struct Reducer {
   double norm(long long n, const double* x, hipStream_t s);  // synchronous
 };
 
-// Right-preconditioned flexible GMRES(restart).  `precond(in, out)` applies
-// the preconditioner (identity if empty).  x holds the initial guess on entry.
-void fgmres(const BsrDev& A, const double* b, double* x, const std::function<void(const double*, double*)>& precond,
-            const KrylovOpts& o, KrylovInfo& info, hipStream_t s);
+// Right-preconditioned flexible GMRES(restart).  x holds the initial guess on
+// entry.
+void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
+            hipStream_t s);
 
 // Right-preconditioned BiCGStab with device-resident scalars (no host round
-// trip per iteration; the recurrence residual is read back every 8
-// iterations).  Convergence is confirmed on the true FP64 residual; a
-// recurrence that converges early or breaks down restarts from it.
+// trip per iteration; the recurrence residual is checked every 8 iterations).
+// Convergence is confirmed on the true FP64 residual; a recurrence that
+// converges early or breaks down restarts from it.
 //
-// ws: null (the solver allocates its vectors), or caller device memory of
-// bicgstab_ws_doubles(n) values, 256-byte aligned, which then holds every
-// vector, scalar and partial sum of the solve (nothing is allocated; the
-// graph option must be off).
-void bicgstab(const BsrDev& A, const double* b, double* x, const std::function<void(const double*, double*)>& precond,
-              const KrylovOpts& o, KrylovInfo& info, hipStream_t s, double* ws = nullptr);
+// kws: the handle's kept workspace (null: one of this call).  ws: null, or
+// caller device memory of bicgstab_ws_doubles(n) values, 256-byte aligned,
+// which then holds every vector, scalar and partial sum of the solve (no
+// device memory is allocated; the graph option must be off).
+void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
+              hipStream_t s, KrylovWs* kws, double* ws = nullptr);
 size_t bicgstab_ws_doubles(long long n);
 
 }  // namespace hfx

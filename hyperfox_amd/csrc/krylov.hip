@@ -210,13 +210,52 @@ __global__ void combine_kernel(long long n, int k, const double* __restrict__ Z,
 }
 
 
+// sum over the block, the same value (and bits) in every thread
+__device__ inline void block_sum2_all(double& a, double& b, double (*red)[RT / 64]) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane == 0) {
+    red[0][wid] = a;
+    red[1][wid] = b;
+  }
+  __syncthreads();
+  a = b = 0.0;
+#pragma unroll
+  for (int w = 0; w < RT / 64; ++w) {
+    a += red[0][w];
+    b += red[1][w];
+  }
+}
+
 // ---------------------------------------------------------------- BiCGStab
 //
-// Scalars live on the device (no host round trip per iteration):
-//   sc[0] rho = (rhat, r)     sc[1] alpha     sc[2] omega     sc[3] rho_prev
-//   sc[4] (rhat, v)           sc[5] (t, s)    sc[6] (t, t)    sc[7] (r, r)
-//   sc[8] breakdown flag (1 when a denominator vanished)
-enum { SC_RHO = 0, SC_ALPHA, SC_OMEGA, SC_RHOP, SC_RV, SC_TS, SC_TT, SC_RR, SC_BRK, SC_N };
+// Scalars live on the device (no host round trip per iteration), in two slots
+// used by even and odd iterations, so that a block that still reads the last
+// iteration's values never races with the block that writes the new ones:
+//   sc[8 par + 0] rho = (rhat, r)   sc[8 par + 1] alpha   sc[8 par + 2] omega
+//   sc[SC_BRK] breakdown flag (1 when a denominator vanished)
+//   sc[SC_STOP] (an int) set by the check kernel: every later kernel returns
+//   at once, so the host may run ahead of the check without changing x
+//   sc[SC_SUMS..+1] reduced partials of a long vector
+// The dot products arrive as one partial per block of the kernel before; each
+// block of the kernel that needs the scalar adds them up again in the same
+// order (a few KB out of L2, behind its own vector loads) instead of waiting
+// for a one-block kernel in between.
+enum { SC_RHO = 0, SC_ALPHA, SC_OMEGA, SC_BRK = 16, SC_STOP = 24, SC_STATUS = 26, SC_SUMS = 28, SC_N = 32 };
+
+__device__ __forceinline__ bool stopped(const double* sc) { return *reinterpret_cast<const int*>(sc + SC_STOP) != 0; }
+
+// the sums of part[0..np) and part[np..2 np), in every thread
+__device__ __forceinline__ void partial_sums(int np, const double* __restrict__ part, bool two, double& d0, double& d1,
+                                             double (*red)[RT / 64]) {
+  d0 = d1 = 0.0;
+  for (int b = threadIdx.x; b < np; b += RT) {
+    d0 += part[b];
+    if (two) d1 += part[np + b];
+  }
+  block_sum2_all(d0, d1, red);
+}
 
 // partial[j * G + blk] = sum over the block's slice of a_j . b_j, j < nd
 __global__ void dots_kernel(long long n, int nd, const double* __restrict__ a0, const double* __restrict__ b0,
@@ -238,76 +277,166 @@ __global__ void dots_kernel(long long n, int nd, const double* __restrict__ a0, 
   }
 }
 
-// Reduce nd partial rows (fixed order) and update the scalars:
-//   op 0: rho_prev = rho; rho = d0; rr = d1          (after the r update)
-//   op 1: rv = d0; alpha = rho / rv                   (after v = A p^)
-//   op 2: ts = d0; tt = d1; omega = ts / tt           (after t = A s^)
-// One workgroup of ST threads; the partials are read ST at a time with
-// several loads in flight per thread.
+// out[j] = sum of partial row j (np values), j < nd, in a fixed order: one
+// workgroup of ST threads, several loads in flight per thread
 constexpr int ST = 1024;
-__global__ __launch_bounds__(ST) void scalars_kernel(int G, int nd, int op, const double* __restrict__ partial,
-                                                     double* __restrict__ sc) {
+__global__ __launch_bounds__(ST) void reduce_partials_kernel(int np, int nd, const double* __restrict__ partial,
+                                                             const double* __restrict__ sc, double* __restrict__ out) {
   __shared__ double red[ST / 64];
-  double d[2] = {0.0, 0.0};
+  if (stopped(sc)) return;
   for (int j = 0; j < nd; ++j) {
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    const double* pj = partial + (size_t)j * G;
+    const double* pj = partial + (size_t)j * np;
     int b = threadIdx.x;
-    for (; b + 3 * ST < G; b += 4 * ST) {
+    for (; b + 3 * ST < np; b += 4 * ST) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) acc[u] += pj[b + u * ST];
     }
-    for (; b < G; b += ST) acc[0] += pj[b];
-    d[j] = block_sum((acc[0] + acc[1]) + (acc[2] + acc[3]), red);
+    for (; b < np; b += ST) acc[0] += pj[b];
+    const double d = block_sum((acc[0] + acc[1]) + (acc[2] + acc[3]), red);
+    if (threadIdx.x == 0) out[j] = d;
     __syncthreads();
   }
-  if (threadIdx.x != 0) return;
-  if (op == 0) {
-    sc[SC_RHOP] = sc[SC_RHO];
-    sc[SC_RHO] = d[0];
-    sc[SC_RR] = d[1];
-    if (d[0] == 0.0) sc[SC_BRK] = 1.0;
-  } else if (op == 1) {
-    sc[SC_RV] = d[0];
-    if (d[0] == 0.0 || !isfinite(d[0])) { sc[SC_BRK] = 1.0; sc[SC_ALPHA] = 0.0; }
-    else sc[SC_ALPHA] = sc[SC_RHO] / d[0];
-  } else {
-    sc[SC_TS] = d[0];
-    sc[SC_TT] = d[1];
-    if (d[1] == 0.0 || !isfinite(d[1])) { sc[SC_BRK] = 1.0; sc[SC_OMEGA] = 0.0; }
-    else sc[SC_OMEGA] = d[0] / d[1];
-    if (sc[SC_OMEGA] == 0.0) sc[SC_BRK] = 1.0;
+}
+
+// Rows of one tile of a vector kernel: with face-block Jacobi fused in
+// (PC_BJACOBI) a tile holds whole face blocks, so that their values meet in LDS.
+template <int PC, int BS>
+constexpr int tile_rows() {
+  return PC == PC_BJACOBI ? (RT / BS) * BS : RT;
+}
+
+// out[t] = (M x)[t] for the tile's value x of row t (in range when on); every
+// thread of the block calls it.  PC_NONE copies, PC_JACOBI scales, PC_BJACOBI
+// multiplies by the block's inverse; any other kind (a preconditioner that
+// runs on its own) leaves out alone.
+template <int PC, int BS>
+__device__ __forceinline__ void apply_tile(bool on, long long t, double x, const double* __restrict__ dinv,
+                                           double* __restrict__ out, double* xs) {
+  if constexpr (PC == PC_NONE) {
+    if (on) out[t] = x;
+  } else if constexpr (PC == PC_JACOBI) {
+    if (on) out[t] = dinv[t] * x;
+  } else if constexpr (PC == PC_BJACOBI) {
+    if (threadIdx.x < tile_rows<PC, BS>()) xs[threadIdx.x] = x;
+    __syncthreads();
+    if (on) out[t] = bsr_row_dot<BS>(dinv + (size_t)t * BS, xs + (threadIdx.x / BS) * BS);
+    __syncthreads();  // xs is refilled by the next tile
   }
 }
 
-// p = r + beta (p - omega v), beta = (rho / rho_prev) (alpha / omega);
-// first = 1: p = r
-__global__ void bicg_p_kernel(long long n, int first, const double* __restrict__ sc, const double* __restrict__ r,
-                              double* __restrict__ p, const double* __restrict__ v) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  if (first) { p[t] = r[t]; return; }
-  const double om = sc[SC_OMEGA], rp = sc[SC_RHOP];
-  const double beta = (rp != 0.0 && om != 0.0) ? (sc[SC_RHO] / rp) * (sc[SC_ALPHA] / om) : 0.0;
-  p[t] = r[t] + beta * (p[t] - om * v[t]);
+// p = r + beta (p - omega v), beta = (rho / rho_prev) (alpha / omega)
+// (first = 1: p = r); p^ = M p.  rho comes from the partials part of
+// (rhat, r), (r, r).
+template <int PC, int BS>
+__global__ __launch_bounds__(RT) void bicg_p_kernel(long long n, int first, int par, int np,
+                                                    const double* __restrict__ part, double* __restrict__ sc,
+                                                    const double* __restrict__ r, double* __restrict__ p,
+                                                    const double* __restrict__ v, const double* __restrict__ dinv,
+                                                    double* __restrict__ ph) {
+  __shared__ double red[2][RT / 64];
+  __shared__ double xs[PC == PC_BJACOBI ? RT : 1];
+  if (stopped(sc)) return;
+  constexpr int TR = tile_rows<PC, BS>();
+  const double* old = sc + 8 * (par ^ 1);
+  const double rp = old[SC_RHO], al = old[SC_ALPHA], om = old[SC_OMEGA];
+  double rho, unused;
+  partial_sums(np, part, false, rho, unused, red);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc[8 * par + SC_RHO] = rho;
+    if (rho == 0.0) sc[SC_BRK] = 1.0;
+  }
+  const double beta = (!first && rp != 0.0 && om != 0.0) ? (rho / rp) * (al / om) : 0.0;
+  for (long long t0 = (long long)blockIdx.x * TR; t0 < n; t0 += (long long)gridDim.x * TR) {
+    const long long t = t0 + threadIdx.x;
+    const bool on = threadIdx.x < TR && t < n;
+    double x = 0.0;
+    if (on) {
+      x = r[t];
+      if (!first) x += beta * (p[t] - om * v[t]);
+      p[t] = x;
+    }
+    apply_tile<PC, BS>(on, t, x, dinv, ph, xs);
+  }
 }
 
-// s = r - alpha v
-__global__ void bicg_s_kernel(long long n, const double* __restrict__ sc, const double* __restrict__ r,
-                              const double* __restrict__ v, double* __restrict__ s) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) s[t] = r[t] - sc[SC_ALPHA] * v[t];
+// alpha = rho / (rhat, v); s = r - alpha v; s^ = M s.  (rhat, v) from part.
+template <int PC, int BS>
+__global__ __launch_bounds__(RT) void bicg_s_kernel(long long n, int par, int np, const double* __restrict__ part,
+                                                    double* __restrict__ sc, const double* __restrict__ r,
+                                                    const double* __restrict__ v, double* __restrict__ s,
+                                                    const double* __restrict__ dinv, double* __restrict__ sh) {
+  __shared__ double red[2][RT / 64];
+  __shared__ double xs[PC == PC_BJACOBI ? RT : 1];
+  if (stopped(sc)) return;
+  constexpr int TR = tile_rows<PC, BS>();
+  double rv, unused;
+  partial_sums(np, part, false, rv, unused, red);
+  const bool bad = rv == 0.0 || !isfinite(rv);
+  const double al = bad ? 0.0 : sc[8 * par + SC_RHO] / rv;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc[8 * par + SC_ALPHA] = al;
+    if (bad) sc[SC_BRK] = 1.0;
+  }
+  for (long long t0 = (long long)blockIdx.x * TR; t0 < n; t0 += (long long)gridDim.x * TR) {
+    const long long t = t0 + threadIdx.x;
+    const bool on = threadIdx.x < TR && t < n;
+    double x = 0.0;
+    if (on) {
+      x = r[t] - al * v[t];
+      s[t] = x;
+    }
+    apply_tile<PC, BS>(on, t, x, dinv, sh, xs);
+  }
 }
 
-// x += alpha p^ + omega s^ ; r = s - omega t
-__global__ void bicg_xr_kernel(long long n, const double* __restrict__ sc, const double* __restrict__ ph,
-                               const double* __restrict__ sh, const double* __restrict__ s,
-                               const double* __restrict__ tv, double* __restrict__ x, double* __restrict__ r) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const double al = sc[SC_ALPHA], om = sc[SC_OMEGA];
-  x[t] += al * ph[t] + om * sh[t];
-  r[t] = s[t] - om * tv[t];
+// omega = (t, s) / (t, t) from part; x += alpha p^ + omega s^; r = s - omega t,
+// with the block partials of rhat . r and r . r in out
+__global__ __launch_bounds__(RT) void bicg_xr_dot_kernel(long long n, int par, int np, const double* __restrict__ part,
+                                                         double* __restrict__ sc, const double* __restrict__ ph,
+                                                         const double* __restrict__ sh, const double* __restrict__ s,
+                                                         const double* __restrict__ tv, const double* __restrict__ rh,
+                                                         double* __restrict__ x, double* __restrict__ r,
+                                                         double* __restrict__ out) {
+  __shared__ double red[2][RT / 64];
+  if (stopped(sc)) return;
+  double ts, tt;
+  partial_sums(np, part, true, ts, tt, red);
+  const bool bad = tt == 0.0 || !isfinite(tt);
+  const double al = sc[8 * par + SC_ALPHA], om = bad ? 0.0 : ts / tt;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc[8 * par + SC_OMEGA] = om;
+    if (om == 0.0) sc[SC_BRK] = 1.0;
+  }
+  double a1 = 0.0, a2 = 0.0;
+  for (long long t = (long long)blockIdx.x * RT + threadIdx.x; t < n; t += (long long)gridDim.x * RT) {
+    x[t] += al * ph[t] + om * sh[t];
+    const double rv = s[t] - om * tv[t];
+    r[t] = rv;
+    a1 += rh[t] * rv;
+    a2 += rv * rv;
+  }
+  __syncthreads();  // red is read above by every thread
+  block_sum2_all(a1, a2, red);
+  if (threadIdx.x == 0) {
+    out[blockIdx.x] = a1;
+    out[gridDim.x + blockIdx.x] = a2;
+  }
+}
+
+// The recurrence residual after an iteration: (rhat, r) and (r, r) from part;
+// sets the stop flag on convergence, a breakdown or a value that is not
+// finite, and reports to the host.
+__global__ __launch_bounds__(RT) void bicg_check_kernel(int np, const double* __restrict__ part, double target, int seq,
+                                                        double* __restrict__ sc, KrylovStatus* __restrict__ st) {
+  __shared__ double red[2][RT / 64];
+  double rho, rr;
+  partial_sums(np, part, true, rho, rr, red);
+  if (threadIdx.x != 0) return;
+  const int code = !isfinite(rr) ? 2 : (sqrt(fabs(rr)) <= target || rho == 0.0 || sc[SC_BRK] != 0.0) ? 1 : 0;
+  *reinterpret_cast<int*>(sc + SC_STOP) = code;
+  __hip_atomic_store(&st->code, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&st->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // y = A x (thread per row) with the block partials of w1 . y (and y . y when
@@ -318,8 +447,9 @@ __global__ __launch_bounds__(RT) void spmv_dot_kernel(int nb, const int* __restr
                                                       const int* __restrict__ col, const double* __restrict__ vals,
                                                       const double* __restrict__ x, double* __restrict__ y,
                                                       const double* __restrict__ w1, int both,
-                                                      double* __restrict__ partial) {
+                                                      const double* __restrict__ sc, double* __restrict__ partial) {
   __shared__ double red[RT / 64];
+  if (stopped(sc)) return;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   double a1 = 0.0, a2 = 0.0;
   if (t < (long long)nb * BS) {
@@ -338,38 +468,8 @@ __global__ __launch_bounds__(RT) void spmv_dot_kernel(int nb, const int* __restr
   }
 }
 
-// x += alpha p^ + omega s^ ; r = s - omega t, with the block partials of
-// rhat . r and r . r
-__global__ __launch_bounds__(RT) void bicg_xr_dot_kernel(long long n, const double* __restrict__ sc,
-                                                         const double* __restrict__ ph, const double* __restrict__ sh,
-                                                         const double* __restrict__ s, const double* __restrict__ tv,
-                                                         const double* __restrict__ rh, double* __restrict__ x,
-                                                         double* __restrict__ r, double* __restrict__ partial) {
-  __shared__ double red[RT / 64];
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  double a1 = 0.0, a2 = 0.0;
-  if (t < n) {
-    const double al = sc[SC_ALPHA], om = sc[SC_OMEGA];
-    x[t] += al * ph[t] + om * sh[t];
-    const double rv = s[t] - om * tv[t];
-    r[t] = rv;
-    a1 = rh[t] * rv;
-    a2 = rv * rv;
-  }
-  const double s1 = block_sum(a1, red);
-  if (threadIdx.x == 0) partial[blockIdx.x] = s1;
-  __syncthreads();
-  const double s2 = block_sum(a2, red);
-  if (threadIdx.x == 0) partial[gridDim.x + blockIdx.x] = s2;
-}
-
 __global__ void set_scalars_kernel(double* __restrict__ sc) {
-  if (threadIdx.x == 0) {
-    for (int i = 0; i < SC_N; ++i) sc[i] = 0.0;
-    sc[SC_ALPHA] = 1.0;
-    sc[SC_OMEGA] = 1.0;
-    sc[SC_RHO] = 1.0;
-  }
+  if (threadIdx.x < SC_N) sc[threadIdx.x] = 0.0;
 }
 
 }  // namespace
@@ -483,8 +583,8 @@ double Reducer::norm(long long n, const double* x, hipStream_t s) {
   return std::sqrt(v);
 }
 
-void fgmres(const BsrDev& A, const double* b, double* x, const std::function<void(const double*, double*)>& precond,
-            const KrylovOpts& o, KrylovInfo& info, hipStream_t s) {
+void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
+            hipStream_t s) {
   const long long n = A.nrows();
   const int m = o.restart;
   if (m < 1 || m > 63) throw std::runtime_error("gmres: restart must be in [1, 63]");
@@ -523,7 +623,7 @@ void fgmres(const BsrDev& A, const double* b, double* x, const std::function<voi
     for (; k < m && it < o.maxits; ++k) {
       double* vk = V.p + (size_t)k * n;
       double* zk = Zb.p + (size_t)k * n;
-      if (precond) precond(vk, zk);
+      if (M.kind != PC_NONE) M.fn(vk, zk);
       else HFX_HIP(hipMemcpyAsync(zk, vk, n * sizeof(double), hipMemcpyDeviceToDevice, s));
       bsr_spmv(A, zk, w.p, nullptr, s);
       // classical Gram-Schmidt, twice
@@ -580,46 +680,76 @@ void fgmres(const BsrDev& A, const double* b, double* x, const std::function<voi
 
 namespace hfx {
 
+KrylovWs::~KrylovWs() {
+  if (status) (void)hipHostFree(status);
+}
+
+KrylovStatus* KrylovWs::host() {
+  if (!status) {
+    void* p = nullptr;
+    HFX_HIP(hipHostMalloc(&p, sizeof(KrylovStatus), hipHostMallocCoherent | hipHostMallocMapped));
+    status = static_cast<KrylovStatus*>(p);
+  }
+  status->seq = -1;
+  status->code = 0;
+  return status;
+}
+
+// Wait until the device has reported `seq` (its kernels are queued on s)
+void KrylovWs::wait(int seq, hipStream_t s) const {
+  for (unsigned spin = 1;; ++spin) {
+    if (__atomic_load_n(&status->seq, __ATOMIC_ACQUIRE) >= seq) return;
+    if ((spin & 0x3ff) == 0) {  // a stream that ended or failed without reporting
+      const hipError_t e = hipStreamQuery(s);
+      if (e == hipErrorNotReady) continue;
+      HFX_HIP(e);
+      if (__atomic_load_n(&status->seq, __ATOMIC_ACQUIRE) >= seq) return;
+      throw std::runtime_error("krylov: the stream ended without a status");
+    }
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+  }
+}
+
 size_t bicgstab_ws_doubles(long long n) {
   const size_t G = (size_t)Reducer::grid_for(n), nblk_rows = (size_t)ceil_div(n, RT);
   return al32(Reducer::doubles(n)) + 8 * al32((size_t)n) + al32(SC_N) + al32(2 * G) + al32(2 * nblk_rows);
 }
 
-void bicgstab(const BsrDev& A, const double* b, double* x, const std::function<void(const double*, double*)>& precond,
-              const KrylovOpts& o, KrylovInfo& info, hipStream_t s, double* ws) {
+// Vectors of up to this many 256-row blocks have their dot products' partials
+// added up again by every block of the next kernel; beyond it a one-block
+// kernel reduces them first.  At the line each of the (at most 512 or 2048)
+// blocks reads 32 KB out of L2, about the time of the extra launch it saves
+// (3.8 us + 2 us of gap on systems of 40,000 to 300,000 rows, where BiCGStab
+// is bound by its launches).
+constexpr int INLINE_PARTIALS = 2048;
+
+void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
+              hipStream_t s, KrylovWs* kws, double* ws) {
   const long long n = A.nrows();
   info = KrylovInfo();
   if (ws && o.graph) throw std::runtime_error("bicgstab: a caller workspace excludes the graph option");
-  Reducer red;
-  const int G = Reducer::grid_for(n);
   const int nblk_rows = ceil_div(n, RT);
-  // r, rhat, p, v, p^, s, s^, t, the device scalars, the dot partials and the
-  // fused-kernel partials: owned buffers, or carved from the caller's memory
-  DevBuf<double> own[11];
+  // r, rhat, p, v, p^, s, s^, t, the device scalars and the partials: carved
+  // from the caller's memory, the handle's kept workspace or a buffer of this
+  // call (systems above the size that is worth keeping)
+  DevBuf<double> own;
+  const size_t need = bicgstab_ws_doubles(n);
+  const bool caller_ws = ws != nullptr;
+  if (!ws) ws = kws ? kws->mem_for(need, own) : (own.alloc(need), own.p);
+  Reducer red;
+  red.init(n, ws);
   double* vec[8];
-  double *sc, *part, *fpart;
-  if (ws) {
-    red.init(n, ws);
-    double* q = ws + al32(Reducer::doubles(n));
-    for (int k = 0; k < 8; ++k, q += al32((size_t)n)) vec[k] = q;
-    sc = q;
-    q += al32(SC_N);
-    part = q;
-    q += al32((size_t)2 * G);
-    fpart = q;
-  } else {
-    red.init(n);
-    for (int k = 0; k < 8; ++k) {
-      own[k].alloc(n);
-      vec[k] = own[k].p;
-    }
-    own[8].alloc(SC_N);
-    own[9].alloc((size_t)2 * G);
-    own[10].alloc((size_t)2 * nblk_rows);
-    sc = own[8].p;
-    part = own[9].p;
-    fpart = own[10].p;
-  }
+  double* q = ws + al32(Reducer::doubles(n));
+  for (int k = 0; k < 8; ++k, q += al32((size_t)n)) vec[k] = q;
+  double* sc = q;
+  double* fpart = q + al32(SC_N);
+  // the x/r update's partials use the reducer's, which is idle meanwhile
+  // (2 x min(8 G, 1024) <= 66 G values)
+  double* xpart = red.partial;
+  const bool inl = nblk_rows <= INLINE_PARTIALS;
+  const int nx = std::min(nblk_rows, inl ? 512 : 1024);
   double *r = vec[0], *rh = vec[1], *p = vec[2], *v = vec[3], *ph = vec[4], *sv = vec[5], *sh = vec[6], *tv = vec[7];
   const double bnorm = red.norm(n, b, s);
   if (bnorm == 0.0) {
@@ -629,23 +759,17 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const std::function<v
     return;
   }
   const double target = o.rtol * bnorm;
-  const int nblk = ceil_div(n, 256);
-  auto apply_M = [&](const double* in, double* out) {
-    if (precond) precond(in, out);
-    else HFX_HIP(hipMemcpyAsync(out, in, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-  };
-  auto dots = [&](int nd, const double* a0, const double* b0, const double* a1, const double* b1, int op) {
-    hipLaunchKernelGGL(dots_kernel, dim3(G), dim3(RT), 0, s, n, nd, a0, b0, a1, b1, part);
-    HFX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(scalars_kernel, dim3(1), dim3(ST), 0, s, G, nd, op, part, sc);
-    HFX_HIP(hipGetLastError());
-  };
-  // fused path: SpMV / update kernels leave one partial per 256-row block
+  // the status of the checks: pinned memory that the host polls, or (nothing
+  // may be allocated) a word of the workspace that it copies
+  KrylovWs local;
+  KrylovWs& hw = kws ? *kws : local;
+  KrylovStatus* st = caller_ws ? reinterpret_cast<KrylovStatus*>(sc + SC_STATUS) : hw.host();
+  int seq = -1;
   auto spmv_dot = [&](const double* xin, double* yout, const double* w1, bool both) {
 #define HFX_BS(B)                                                                                          \
   case B:                                                                                                  \
     hipLaunchKernelGGL((spmv_dot_kernel<B>), dim3(nblk_rows), dim3(RT), 0, s, A.nb, A.rowptr.p, A.col.p,   \
-                       A.vals.p, xin, yout, w1, both ? 1 : 0, fpart);                                    \
+                       A.vals.p, xin, yout, w1, both ? 1 : 0, sc, fpart);                                 \
     break;
     switch (A.bs) {
       HFX_BS(1) HFX_BS(2) HFX_BS(3) HFX_BS(4) HFX_BS(5) HFX_BS(6) HFX_BS(7) HFX_BS(8) HFX_BS(9) HFX_BS(10) HFX_BS(11) HFX_BS(12) HFX_BS(15) HFX_BS(18) HFX_BS(21) HFX_BS(30)
@@ -653,30 +777,62 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const std::function<v
     }
 #undef HFX_BS
     HFX_HIP(hipGetLastError());
+    if (!inl) {
+      hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(ST), 0, s, nblk_rows, both ? 2 : 1, fpart, sc,
+                         sc + SC_SUMS);
+      HFX_HIP(hipGetLastError());
+    }
   };
-  auto scalars = [&](int nd, int op) {
-    hipLaunchKernelGGL(scalars_kernel, dim3(1), dim3(ST), 0, s, nblk_rows, nd, op, fpart, sc);
+  const int np = inl ? nblk_rows : 1;
+  const double* part = inl ? fpart : sc + SC_SUMS;
+  // the vector kernels with the preconditioner fused in (point and block Jacobi) or followed by its own kernels
+  const int tiles = M.kind == PC_BJACOBI ? ceil_div(n, (RT / A.bs) * A.bs) : nblk_rows;
+  const int vgrid = inl ? std::min(tiles, 2048) : tiles;
+  auto pstep = [&](int first, int par) {
+#define HFX_LAUNCH(PC, B)                                                                                           \
+  hipLaunchKernelGGL((bicg_p_kernel<PC, B>), dim3(vgrid), dim3(RT), 0, s, n, first, par, nx, xpart, sc, r, p, v, \
+                     M.dinv, ph)
+#define HFX_BS(B) case B: HFX_LAUNCH(PC_BJACOBI, B); break;
+    if (M.kind == PC_NONE) HFX_LAUNCH(PC_NONE, 1);
+    else if (M.kind == PC_JACOBI) HFX_LAUNCH(PC_JACOBI, 1);
+    else if (M.kind != PC_BJACOBI) HFX_LAUNCH(PC_OTHER, 1);
+    else switch (A.bs) {
+      HFX_BS(1) HFX_BS(2) HFX_BS(3) HFX_BS(4) HFX_BS(5) HFX_BS(6) HFX_BS(7) HFX_BS(8) HFX_BS(9) HFX_BS(10) HFX_BS(11) HFX_BS(12) HFX_BS(15) HFX_BS(18) HFX_BS(21) HFX_BS(30)
+      default: throw std::runtime_error("bicgstab: unsupported block size");
+    }
+#undef HFX_BS
+#undef HFX_LAUNCH
     HFX_HIP(hipGetLastError());
+    if (M.kind == PC_OTHER) M.fn(p, ph);
+  };
+  auto sstep = [&](int par) {
+#define HFX_LAUNCH(PC, B)                                                                                           \
+  hipLaunchKernelGGL((bicg_s_kernel<PC, B>), dim3(vgrid), dim3(RT), 0, s, n, par, np, part, sc, r, v, sv, M.dinv, sh)
+#define HFX_BS(B) case B: HFX_LAUNCH(PC_BJACOBI, B); break;
+    if (M.kind == PC_NONE) HFX_LAUNCH(PC_NONE, 1);
+    else if (M.kind == PC_JACOBI) HFX_LAUNCH(PC_JACOBI, 1);
+    else if (M.kind != PC_BJACOBI) HFX_LAUNCH(PC_OTHER, 1);
+    else switch (A.bs) {
+      HFX_BS(1) HFX_BS(2) HFX_BS(3) HFX_BS(4) HFX_BS(5) HFX_BS(6) HFX_BS(7) HFX_BS(8) HFX_BS(9) HFX_BS(10) HFX_BS(11) HFX_BS(12) HFX_BS(15) HFX_BS(18) HFX_BS(21) HFX_BS(30)
+      default: throw std::runtime_error("bicgstab: unsupported block size");
+    }
+#undef HFX_BS
+#undef HFX_LAUNCH
+    HFX_HIP(hipGetLastError());
+    if (M.kind == PC_OTHER) M.fn(sv, sh);
   };
   const int check_every = 8;
-  // one steady iteration (after the first of a restart): p, M p, A p^ with
+  // one iteration (first: the one after a restart): p, M p, A p^ with
   // (rhat, v), alpha, s, M s, A s^ with (s, t) and (t, t), omega, x, r with
   // (rhat, r) and (r, r)
-  auto steady = [&]() {
-    hipLaunchKernelGGL(bicg_p_kernel, dim3(nblk), dim3(256), 0, s, n, 0, sc, r, p, v);
-    HFX_HIP(hipGetLastError());
-    apply_M(p, ph);
+  auto iteration = [&](int first, int par) {
+    pstep(first, par);
     spmv_dot(ph, v, rh, false);
-    scalars(1, 1);
-    hipLaunchKernelGGL(bicg_s_kernel, dim3(nblk), dim3(256), 0, s, n, sc, r, v, sv);
-    HFX_HIP(hipGetLastError());
-    apply_M(sv, sh);
+    sstep(par);
     spmv_dot(sh, tv, sv, true);
-    scalars(2, 2);
-    hipLaunchKernelGGL(bicg_xr_dot_kernel, dim3(nblk), dim3(RT), 0, s, n, sc, ph, sh, sv, tv, rh, x, r,
-                       fpart);
+    hipLaunchKernelGGL(bicg_xr_dot_kernel, dim3(nx), dim3(RT), 0, s, n, par, np, part, sc, ph, sh, sv, tv, rh, x, r,
+                       xpart);
     HFX_HIP(hipGetLastError());
-    scalars(2, 0);
   };
   // check_every steady iterations as one graph, captured at first use; it
   // holds kernels only (no memset or copy nodes), and every buffer it names
@@ -689,12 +845,12 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const std::function<v
       if (g) (void)hipGraphDestroy(g);
     }
   } gh;
-  const bool use_graph = o.graph && static_cast<bool>(precond);
+  const bool use_graph = o.graph && M.kind != PC_NONE;
   auto graph_block = [&]() {
     if (!gh.e) {
       HFX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       try {
-        for (int k = 0; k < check_every; ++k) steady();
+        for (int k = 0; k < check_every; ++k) iteration(0, k & 1);
       } catch (...) {
         hipGraph_t g = nullptr;
         (void)hipStreamEndCapture(s, &g);
@@ -707,61 +863,57 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const std::function<v
     HFX_HIP(hipGraphLaunch(gh.e, s));
   };
   int it = 0;
-  bool restart = true;
   while (true) {
-    if (!restart && use_graph && it % check_every == 0 && it + check_every <= o.maxits) {
-      graph_block();
-      it += check_every;
-      double hs[SC_N];
-      HFX_HIP(hipMemcpyAsync(hs, sc, sizeof(hs), hipMemcpyDeviceToHost, s));
-      HFX_HIP(hipStreamSynchronize(s));
-      const double rr = std::sqrt(std::fabs(hs[SC_RR]));
-      if (!std::isfinite(hs[SC_RR])) { info.reason = DIVERGED_NANORINF; break; }
-      if (rr <= target || hs[SC_BRK] != 0.0 || it >= o.maxits) restart = true;
-      continue;
-    }
-    if (restart) {
-      // r = b - A x (true FP64 residual), rhat = r, rho = (r, r)
-      bsr_spmv(A, x, r, b, s);
-      const double rn = red.norm(n, r, s);
-      info.true_relres = rn / bnorm;
-      if (!std::isfinite(rn)) { info.reason = DIVERGED_NANORINF; break; }
-      if (rn <= target) { info.reason = CONVERGED_RTOL; break; }
-      if (it >= o.maxits) { info.reason = DIVERGED_ITS; break; }
-      HFX_HIP(hipMemcpyAsync(rh, r, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-      hipLaunchKernelGGL(set_scalars_kernel, dim3(1), dim3(64), 0, s, sc);
+    // r = b - A x (true FP64 residual), rhat = r, rho = (r, r)
+    bsr_spmv(A, x, r, b, s);
+    const double rn = red.norm(n, r, s);
+    info.true_relres = rn / bnorm;
+    if (!std::isfinite(rn)) { info.reason = DIVERGED_NANORINF; break; }
+    if (rn <= target) { info.reason = CONVERGED_RTOL; break; }
+    if (it >= o.maxits) { info.reason = DIVERGED_ITS; break; }
+    HFX_HIP(hipMemcpyAsync(rh, r, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL(set_scalars_kernel, dim3(1), dim3(64), 0, s, sc);
+    HFX_HIP(hipGetLastError());
+    hipLaunchKernelGGL(dots_kernel, dim3(nx), dim3(RT), 0, s, n, 2, rh, r, r, r, xpart);
+    HFX_HIP(hipGetLastError());
+    ++info.restarts;
+    // Iterations up to the next restart.  The recurrence residual is checked
+    // every check_every iterations; one iteration is queued behind each check
+    // before its result is awaited (it does nothing once the check has set the
+    // stop flag), so the device does not idle meanwhile.
+    bool first = true;
+    int code = 0, ahead = 0;
+    while (true) {
+      if (ahead) {
+        ahead = 0;  // already queued
+        ++it;
+      } else if (!first && use_graph && it % check_every == 0 && it + check_every <= o.maxits) {
+        graph_block();
+        it += check_every;
+      } else {
+        iteration(first ? 1 : 0, it & 1);
+        first = false;
+        ++it;
+      }
+      if (it % check_every != 0 && it < o.maxits) continue;
+      hipLaunchKernelGGL(bicg_check_kernel, dim3(1), dim3(RT), 0, s, nx, xpart, target, ++seq, sc, st);
       HFX_HIP(hipGetLastError());
-      dots(2, rh, r, r, r, 0);
-      ++info.restarts;
-      restart = false;
-      hipLaunchKernelGGL(bicg_p_kernel, dim3(nblk), dim3(256), 0, s, n, 1, sc, r, p, v);
-      HFX_HIP(hipGetLastError());
-      apply_M(p, ph);
-      spmv_dot(ph, v, rh, false);          // v = A p^, (rhat, v)
-      scalars(1, 1);
-      hipLaunchKernelGGL(bicg_s_kernel, dim3(nblk), dim3(256), 0, s, n, sc, r, v, sv);
-      HFX_HIP(hipGetLastError());
-      apply_M(sv, sh);
-      spmv_dot(sh, tv, sv, true);          // t = A s^, (s, t), (t, t)
-      scalars(2, 2);
-      hipLaunchKernelGGL(bicg_xr_dot_kernel, dim3(nblk), dim3(RT), 0, s, n, sc, ph, sh, sv, tv, rh, x,
-                         r, fpart);
-      HFX_HIP(hipGetLastError());
-      scalars(2, 0);                             // (rhat, r), (r, r)
-    } else {
-      steady();
-    }
-    ++it;
-    if (it % check_every == 0 || it >= o.maxits) {
-      double hs[SC_N];
-      HFX_HIP(hipMemcpyAsync(hs, sc, sizeof(hs), hipMemcpyDeviceToHost, s));
-      HFX_HIP(hipStreamSynchronize(s));
-      const double rr = std::sqrt(std::fabs(hs[SC_RR]));
-      if (!std::isfinite(hs[SC_RR])) { info.reason = DIVERGED_NANORINF; break; }
+      if (caller_ws) {
+        HFX_HIP(hipMemcpyAsync(&code, &st->code, sizeof(int), hipMemcpyDeviceToHost, s));
+        HFX_HIP(hipStreamSynchronize(s));
+      } else {
+        if (!use_graph && it < o.maxits) {
+          iteration(0, it & 1);
+          ahead = 1;
+        }
+        hw.wait(seq, s);
+        code = __atomic_load_n(&st->code, __ATOMIC_RELAXED);
+      }
       // converged recurrence, breakdown, or the iteration budget: restart from
       // (and test) the true residual; maxits bounds the number of restarts
-      if (rr <= target || hs[SC_BRK] != 0.0 || it >= o.maxits) restart = true;
+      if (code != 0 || it >= o.maxits) break;
     }
+    if (code == 2) { info.reason = DIVERGED_NANORINF; break; }
   }
   info.iters = it;
   HFX_HIP(hipStreamSynchronize(s));

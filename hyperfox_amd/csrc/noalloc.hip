@@ -93,13 +93,17 @@ extern "C" int hfx_hdg_solve_noalloc(hfx_hdg* h, int pc, double rtol, int maxits
     double* dinv = ws + need_k;
     hipStream_t s = h->stream;
     // the preconditioners of hfx_hdg_solve, their inverse diagonal in the workspace
-    std::function<void(const double*, double*)> M;
+    hfx::PcApply M;
     if (pc == HFX_PC_JACOBI) {
       hfx::bsr_inv_point_diag(A, dinv, s);
-      M = [n, dinv, s](const double* in, double* out) { hfx::apply_point_diag(n, dinv, in, out, s); };
+      M.kind = hfx::PC_JACOBI;
+      M.dinv = dinv;
+      M.fn = [n, dinv, s](const double* in, double* out) { hfx::apply_point_diag(n, dinv, in, out, s); };
     } else if (pc == HFX_PC_BJACOBI) {
       hfx::bsr_invert_diag(A, dinv, s);
-      M = [&A, dinv, s](const double* in, double* out) { hfx::apply_block_diag(A.nb, A.bs, dinv, in, out, s); };
+      M.kind = hfx::PC_BJACOBI;
+      M.dinv = dinv;
+      M.fn = [&A, dinv, s](const double* in, double* out) { hfx::apply_block_diag(A.nb, A.bs, dinv, in, out, s); };
     }
     HFX_HIP(hipMemsetAsync(h->lambda.p, 0, n * sizeof(double), s));  // zero initial guess, as PETSc
     hfx::KrylovOpts o;
@@ -107,7 +111,7 @@ extern "C" int hfx_hdg_solve_noalloc(hfx_hdg* h, int pc, double rtol, int maxits
     o.maxits = maxits;
     o.graph = false;
     hfx::KrylovInfo ki;
-    hfx::bicgstab(A, h->rhs.p, h->lambda.p, M, o, ki, s, ws);
+    hfx::bicgstab(A, h->rhs.p, h->lambda.p, M, o, ki, s, &h->kws, ws);
     const hfx::Mesh& m = h->mesh;
     hfx::launch_reconstruct(m.nCells, m.nN, m.nN * h->dim, m.nFpc, m.nNf, h->U.p, h->U0.p, h->Q.p, h->Q0.p, h->c2f.p,
                             h->perm.p, h->lambda.p, h->u.p, h->q.p, s);
