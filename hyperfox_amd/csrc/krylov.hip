@@ -11,10 +11,30 @@ namespace {
 
 constexpr int RT = 256;  // reduction block size
 
-__device__ inline double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+// value of v, CTRL & 15 lanes to the right in its row of 16 (DPP row_shl)
+template <int CTRL>
+__device__ __forceinline__ double row_shl(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+// sum over the wavefront, valid in lane 0: the tree of lane distances 32, 16,
+// 8, .., 1, the steps inside a row of 16 lanes as DPP moves
+__device__ __forceinline__ double wave_sum(double v) {
+  v += __shfl_down(v, 32, 64);
+  v += __shfl_down(v, 16, 64);
+  v += row_shl<0x108>(v);
+  v += row_shl<0x104>(v);
+  v += row_shl<0x102>(v);
+  v += row_shl<0x101>(v);
   return v;
 }
+
+// Partials of one dot product are added up by SV = 1024 (real or virtual)
+// threads, strided, then wave by wave: the same order, and so the same bits,
+// in the one-block kernel (reduce_partials_kernel) and in partial_sums below.
+constexpr int SV = 1024;
 
 // block-wide sum, result valid in thread 0
 __device__ inline double block_sum(double v, double* red) {
@@ -210,24 +230,6 @@ __global__ void combine_kernel(long long n, int k, const double* __restrict__ Z,
 }
 
 
-// sum over the block, the same value (and bits) in every thread
-__device__ inline void block_sum2_all(double& a, double& b, double (*red)[RT / 64]) {
-  a = wave_sum(a);
-  b = wave_sum(b);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) {
-    red[0][wid] = a;
-    red[1][wid] = b;
-  }
-  __syncthreads();
-  a = b = 0.0;
-#pragma unroll
-  for (int w = 0; w < RT / 64; ++w) {
-    a += red[0][w];
-    b += red[1][w];
-  }
-}
-
 // ---------------------------------------------------------------- BiCGStab
 //
 // Scalars live on the device (no host round trip per iteration), in two slots
@@ -237,24 +239,54 @@ __device__ inline void block_sum2_all(double& a, double& b, double (*red)[RT / 6
 //   sc[SC_BRK] breakdown flag (1 when a denominator vanished)
 //   sc[SC_STOP] (an int) set by the check kernel: every later kernel returns
 //   at once, so the host may run ahead of the check without changing x
-//   sc[SC_SUMS..+1] reduced partials of a long vector
+//   sc[SC_SUMS..+1], sc[SC_XSUMS..+1] reduced partials of a long vector (the
+//   products with A, the x/r update)
 // The dot products arrive as one partial per block of the kernel before; each
 // block of the kernel that needs the scalar adds them up again in the same
 // order (a few KB out of L2, behind its own vector loads) instead of waiting
 // for a one-block kernel in between.
-enum { SC_RHO = 0, SC_ALPHA, SC_OMEGA, SC_BRK = 16, SC_STOP = 24, SC_STATUS = 26, SC_SUMS = 28, SC_N = 32 };
+enum { SC_RHO = 0, SC_ALPHA, SC_OMEGA, SC_BRK = 16, SC_STOP = 24, SC_STATUS = 26, SC_XSUMS = 28, SC_SUMS = 30, SC_N = 32 };
 
 __device__ __forceinline__ bool stopped(const double* sc) { return *reinterpret_cast<const int*>(sc + SC_STOP) != 0; }
 
-// the sums of part[0..np) and part[np..2 np), in every thread
+// The sums of part[0..np) and (two) part[np..2 np), np <= 2 SV, in every
+// thread; each of the RT threads stands for SV / RT threads of the one-block
+// kernel.
 __device__ __forceinline__ void partial_sums(int np, const double* __restrict__ part, bool two, double& d0, double& d1,
-                                             double (*red)[RT / 64]) {
-  d0 = d1 = 0.0;
-  for (int b = threadIdx.x; b < np; b += RT) {
-    d0 += part[b];
-    if (two) d1 += part[np + b];
+                                             double (*red)[SV / 64]) {
+  constexpr int NV = SV / RT;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  // every load in flight at once, then the NV (or 2 NV) independent trees
+  double a[NV], c[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int b = v * RT + threadIdx.x;
+    a[v] = b < np ? part[b] : 0.0;
+    c[v] = two && b < np ? part[np + b] : 0.0;
+    if (np > SV) {
+      a[v] += b + SV < np ? part[b + SV] : 0.0;
+      c[v] += two && b + SV < np ? part[np + b + SV] : 0.0;
+    }
   }
-  block_sum2_all(d0, d1, red);
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    if (v * RT >= np) break;  // the rest are zeros
+    a[v] = wave_sum(a[v]);
+    if (two) c[v] = wave_sum(c[v]);
+  }
+  if (lane == 0)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      red[0][v * (RT / 64) + wid] = a[v];
+      red[1][v * (RT / 64) + wid] = c[v];
+    }
+  __syncthreads();
+  d0 = d1 = 0.0;
+  const int nw = min(NV, (np + RT - 1) / RT) * (RT / 64);
+  for (int w = 0; w < nw; ++w) {
+    d0 += red[0][w];
+    if (two) d1 += red[1][w];
+  }
 }
 
 // partial[j * G + blk] = sum over the block's slice of a_j . b_j, j < nd
@@ -277,22 +309,21 @@ __global__ void dots_kernel(long long n, int nd, const double* __restrict__ a0, 
   }
 }
 
-// out[j] = sum of partial row j (np values), j < nd, in a fixed order: one
-// workgroup of ST threads, several loads in flight per thread
-constexpr int ST = 1024;
-__global__ __launch_bounds__(ST) void reduce_partials_kernel(int np, int nd, const double* __restrict__ partial,
+// out[j] = sum of partial row j (np values), j < nd: one workgroup of SV
+// threads, several loads in flight per thread
+__global__ __launch_bounds__(SV) void reduce_partials_kernel(int np, int nd, const double* __restrict__ partial,
                                                              const double* __restrict__ sc, double* __restrict__ out) {
-  __shared__ double red[ST / 64];
+  __shared__ double red[SV / 64];
   if (stopped(sc)) return;
   for (int j = 0; j < nd; ++j) {
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     const double* pj = partial + (size_t)j * np;
     int b = threadIdx.x;
-    for (; b + 3 * ST < np; b += 4 * ST) {
+    for (; b + 3 * SV < np; b += 4 * SV) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc[u] += pj[b + u * ST];
+      for (int u = 0; u < 4; ++u) acc[u] += pj[b + u * SV];
     }
-    for (; b < np; b += ST) acc[0] += pj[b];
+    for (; b < np; b += SV) acc[0] += pj[b];
     const double d = block_sum((acc[0] + acc[1]) + (acc[2] + acc[3]), red);
     if (threadIdx.x == 0) out[j] = d;
     __syncthreads();
@@ -321,7 +352,6 @@ __device__ __forceinline__ void apply_tile(bool on, long long t, double x, const
     if (threadIdx.x < tile_rows<PC, BS>()) xs[threadIdx.x] = x;
     __syncthreads();
     if (on) out[t] = bsr_row_dot<BS>(dinv + (size_t)t * BS, xs + (threadIdx.x / BS) * BS);
-    __syncthreads();  // xs is refilled by the next tile
   }
 }
 
@@ -334,10 +364,20 @@ __global__ __launch_bounds__(RT) void bicg_p_kernel(long long n, int first, int 
                                                     const double* __restrict__ r, double* __restrict__ p,
                                                     const double* __restrict__ v, const double* __restrict__ dinv,
                                                     double* __restrict__ ph) {
-  __shared__ double red[2][RT / 64];
+  __shared__ double red[2][SV / 64];
   __shared__ double xs[PC == PC_BJACOBI ? RT : 1];
   if (stopped(sc)) return;
   constexpr int TR = tile_rows<PC, BS>();
+  const long long t = (long long)blockIdx.x * TR + threadIdx.x;
+  const bool on = threadIdx.x < TR && t < n;
+  double x = 0.0, pv = 0.0, vv = 0.0;  // on their way while the partials are added up
+  if (on) {
+    x = r[t];
+    if (!first) {
+      pv = p[t];
+      vv = v[t];
+    }
+  }
   const double* old = sc + 8 * (par ^ 1);
   const double rp = old[SC_RHO], al = old[SC_ALPHA], om = old[SC_OMEGA];
   double rho, unused;
@@ -347,17 +387,9 @@ __global__ __launch_bounds__(RT) void bicg_p_kernel(long long n, int first, int 
     if (rho == 0.0) sc[SC_BRK] = 1.0;
   }
   const double beta = (!first && rp != 0.0 && om != 0.0) ? (rho / rp) * (al / om) : 0.0;
-  for (long long t0 = (long long)blockIdx.x * TR; t0 < n; t0 += (long long)gridDim.x * TR) {
-    const long long t = t0 + threadIdx.x;
-    const bool on = threadIdx.x < TR && t < n;
-    double x = 0.0;
-    if (on) {
-      x = r[t];
-      if (!first) x += beta * (p[t] - om * v[t]);
-      p[t] = x;
-    }
-    apply_tile<PC, BS>(on, t, x, dinv, ph, xs);
-  }
+  if (!first) x += beta * (pv - om * vv);
+  if (on) p[t] = x;
+  apply_tile<PC, BS>(on, t, x, dinv, ph, xs);
 }
 
 // alpha = rho / (rhat, v); s = r - alpha v; s^ = M s.  (rhat, v) from part.
@@ -366,10 +398,13 @@ __global__ __launch_bounds__(RT) void bicg_s_kernel(long long n, int par, int np
                                                     double* __restrict__ sc, const double* __restrict__ r,
                                                     const double* __restrict__ v, double* __restrict__ s,
                                                     const double* __restrict__ dinv, double* __restrict__ sh) {
-  __shared__ double red[2][RT / 64];
+  __shared__ double red[2][SV / 64];
   __shared__ double xs[PC == PC_BJACOBI ? RT : 1];
   if (stopped(sc)) return;
   constexpr int TR = tile_rows<PC, BS>();
+  const long long t = (long long)blockIdx.x * TR + threadIdx.x;
+  const bool on = threadIdx.x < TR && t < n;
+  const double rt = on ? r[t] : 0.0, vt = on ? v[t] : 0.0;
   double rv, unused;
   partial_sums(np, part, false, rv, unused, red);
   const bool bad = rv == 0.0 || !isfinite(rv);
@@ -378,16 +413,9 @@ __global__ __launch_bounds__(RT) void bicg_s_kernel(long long n, int par, int np
     sc[8 * par + SC_ALPHA] = al;
     if (bad) sc[SC_BRK] = 1.0;
   }
-  for (long long t0 = (long long)blockIdx.x * TR; t0 < n; t0 += (long long)gridDim.x * TR) {
-    const long long t = t0 + threadIdx.x;
-    const bool on = threadIdx.x < TR && t < n;
-    double x = 0.0;
-    if (on) {
-      x = r[t] - al * v[t];
-      s[t] = x;
-    }
-    apply_tile<PC, BS>(on, t, x, dinv, sh, xs);
-  }
+  const double x = rt - al * vt;
+  if (on) s[t] = x;
+  apply_tile<PC, BS>(on, t, x, dinv, sh, xs);
 }
 
 // omega = (t, s) / (t, t) from part; x += alpha p^ + omega s^; r = s - omega t,
@@ -398,8 +426,19 @@ __global__ __launch_bounds__(RT) void bicg_xr_dot_kernel(long long n, int par, i
                                                          const double* __restrict__ tv, const double* __restrict__ rh,
                                                          double* __restrict__ x, double* __restrict__ r,
                                                          double* __restrict__ out) {
-  __shared__ double red[2][RT / 64];
+  __shared__ double red[2][SV / 64];
   if (stopped(sc)) return;
+  const long long t = (long long)blockIdx.x * RT + threadIdx.x;
+  const bool on = t < n;
+  double xv = 0.0, pv = 0.0, hv = 0.0, sv = 0.0, tt_ = 0.0, rhv = 0.0;
+  if (on) {
+    xv = x[t];
+    pv = ph[t];
+    hv = sh[t];
+    sv = s[t];
+    tt_ = tv[t];
+    rhv = rh[t];
+  }
   double ts, tt;
   partial_sums(np, part, true, ts, tt, red);
   const bool bad = tt == 0.0 || !isfinite(tt);
@@ -409,19 +448,19 @@ __global__ __launch_bounds__(RT) void bicg_xr_dot_kernel(long long n, int par, i
     if (om == 0.0) sc[SC_BRK] = 1.0;
   }
   double a1 = 0.0, a2 = 0.0;
-  for (long long t = (long long)blockIdx.x * RT + threadIdx.x; t < n; t += (long long)gridDim.x * RT) {
-    x[t] += al * ph[t] + om * sh[t];
-    const double rv = s[t] - om * tv[t];
+  if (on) {
+    x[t] = xv + (al * pv + om * hv);
+    const double rv = sv - om * tt_;
     r[t] = rv;
-    a1 += rh[t] * rv;
-    a2 += rv * rv;
+    a1 = rhv * rv;
+    a2 = rv * rv;
   }
-  __syncthreads();  // red is read above by every thread
-  block_sum2_all(a1, a2, red);
-  if (threadIdx.x == 0) {
-    out[blockIdx.x] = a1;
-    out[gridDim.x + blockIdx.x] = a2;
-  }
+  __shared__ double red1[RT / 64];
+  const double s1 = block_sum(a1, red1);
+  if (threadIdx.x == 0) out[blockIdx.x] = s1;
+  __syncthreads();
+  const double s2 = block_sum(a2, red1);
+  if (threadIdx.x == 0) out[gridDim.x + blockIdx.x] = s2;
 }
 
 // The recurrence residual after an iteration: (rhat, r) and (r, r) from part;
@@ -429,7 +468,7 @@ __global__ __launch_bounds__(RT) void bicg_xr_dot_kernel(long long n, int par, i
 // finite, and reports to the host.
 __global__ __launch_bounds__(RT) void bicg_check_kernel(int np, const double* __restrict__ part, double target, int seq,
                                                         double* __restrict__ sc, KrylovStatus* __restrict__ st) {
-  __shared__ double red[2][RT / 64];
+  __shared__ double red[2][SV / 64];
   double rho, rr;
   partial_sums(np, part, true, rho, rr, red);
   if (threadIdx.x != 0) return;
@@ -719,8 +758,8 @@ size_t bicgstab_ws_doubles(long long n) {
 
 // Vectors of up to this many 256-row blocks have their dot products' partials
 // added up again by every block of the next kernel; beyond it a one-block
-// kernel reduces them first.  At the line each of the (at most 512 or 2048)
-// blocks reads 32 KB out of L2, about the time of the extra launch it saves
+// kernel reduces them first.  At the line each of the (at most 2048) blocks
+// reads 32 KB out of L2, about the time of the extra launch it saves
 // (3.8 us + 2 us of gap on systems of 40,000 to 300,000 rows, where BiCGStab
 // is bound by its launches).
 constexpr int INLINE_PARTIALS = 2048;
@@ -745,11 +784,11 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, con
   for (int k = 0; k < 8; ++k, q += al32((size_t)n)) vec[k] = q;
   double* sc = q;
   double* fpart = q + al32(SC_N);
-  // the x/r update's partials use the reducer's, which is idle meanwhile
-  // (2 x min(8 G, 1024) <= 66 G values)
-  double* xpart = red.partial;
+  // the x/r update's partials use the reducer's, which is idle meanwhile, on
+  // systems that keep them (2 x 8 G <= 66 G values), and fpart on larger ones,
+  // where they are reduced at once
   const bool inl = nblk_rows <= INLINE_PARTIALS;
-  const int nx = std::min(nblk_rows, inl ? 512 : 1024);
+  double* xpart = inl ? red.partial : fpart;
   double *r = vec[0], *rh = vec[1], *p = vec[2], *v = vec[3], *ph = vec[4], *sv = vec[5], *sh = vec[6], *tv = vec[7];
   const double bnorm = red.norm(n, b, s);
   if (bnorm == 0.0) {
@@ -765,6 +804,10 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, con
   KrylovWs& hw = kws ? *kws : local;
   KrylovStatus* st = caller_ws ? reinterpret_cast<KrylovStatus*>(sc + SC_STATUS) : hw.host();
   int seq = -1;
+  auto reduce = [&](int count, int nd, const double* from, double* to) {
+    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(SV), 0, s, count, nd, from, sc, to);
+    HFX_HIP(hipGetLastError());
+  };
   auto spmv_dot = [&](const double* xin, double* yout, const double* w1, bool both) {
 #define HFX_BS(B)                                                                                          \
   case B:                                                                                                  \
@@ -777,20 +820,18 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, con
     }
 #undef HFX_BS
     HFX_HIP(hipGetLastError());
-    if (!inl) {
-      hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(ST), 0, s, nblk_rows, both ? 2 : 1, fpart, sc,
-                         sc + SC_SUMS);
-      HFX_HIP(hipGetLastError());
-    }
+    if (!inl) reduce(nblk_rows, both ? 2 : 1, fpart, sc + SC_SUMS);
   };
   const int np = inl ? nblk_rows : 1;
   const double* part = inl ? fpart : sc + SC_SUMS;
+  const double* xsums = inl ? xpart : sc + SC_XSUMS;  // (rhat, r), (r, r): np values each
   // the vector kernels with the preconditioner fused in (point and block Jacobi) or followed by its own kernels
   const int tiles = M.kind == PC_BJACOBI ? ceil_div(n, (RT / A.bs) * A.bs) : nblk_rows;
-  const int vgrid = inl ? std::min(tiles, 2048) : tiles;
   auto pstep = [&](int first, int par) {
+    const int fnp = first ? 1 : np;
+    const double* fpt = first ? sc + SC_XSUMS : xsums;
 #define HFX_LAUNCH(PC, B)                                                                                           \
-  hipLaunchKernelGGL((bicg_p_kernel<PC, B>), dim3(vgrid), dim3(RT), 0, s, n, first, par, nx, xpart, sc, r, p, v, \
+  hipLaunchKernelGGL((bicg_p_kernel<PC, B>), dim3(tiles), dim3(RT), 0, s, n, first, par, fnp, fpt, sc, r, p, v, \
                      M.dinv, ph)
 #define HFX_BS(B) case B: HFX_LAUNCH(PC_BJACOBI, B); break;
     if (M.kind == PC_NONE) HFX_LAUNCH(PC_NONE, 1);
@@ -807,7 +848,7 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, con
   };
   auto sstep = [&](int par) {
 #define HFX_LAUNCH(PC, B)                                                                                           \
-  hipLaunchKernelGGL((bicg_s_kernel<PC, B>), dim3(vgrid), dim3(RT), 0, s, n, par, np, part, sc, r, v, sv, M.dinv, sh)
+  hipLaunchKernelGGL((bicg_s_kernel<PC, B>), dim3(tiles), dim3(RT), 0, s, n, par, np, part, sc, r, v, sv, M.dinv, sh)
 #define HFX_BS(B) case B: HFX_LAUNCH(PC_BJACOBI, B); break;
     if (M.kind == PC_NONE) HFX_LAUNCH(PC_NONE, 1);
     else if (M.kind == PC_JACOBI) HFX_LAUNCH(PC_JACOBI, 1);
@@ -830,9 +871,10 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, con
     spmv_dot(ph, v, rh, false);
     sstep(par);
     spmv_dot(sh, tv, sv, true);
-    hipLaunchKernelGGL(bicg_xr_dot_kernel, dim3(nx), dim3(RT), 0, s, n, par, np, part, sc, ph, sh, sv, tv, rh, x, r,
-                       xpart);
+    hipLaunchKernelGGL(bicg_xr_dot_kernel, dim3(nblk_rows), dim3(RT), 0, s, n, par, np, part, sc, ph, sh, sv, tv, rh,
+                       x, r, xpart);
     HFX_HIP(hipGetLastError());
+    if (!inl) reduce(nblk_rows, 2, xpart, sc + SC_XSUMS);
   };
   // check_every steady iterations as one graph, captured at first use; it
   // holds kernels only (no memset or copy nodes), and every buffer it names
@@ -874,8 +916,9 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, con
     HFX_HIP(hipMemcpyAsync(rh, r, n * sizeof(double), hipMemcpyDeviceToDevice, s));
     hipLaunchKernelGGL(set_scalars_kernel, dim3(1), dim3(64), 0, s, sc);
     HFX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(dots_kernel, dim3(nx), dim3(RT), 0, s, n, 2, rh, r, r, r, xpart);
+    hipLaunchKernelGGL(dots_kernel, dim3(red.grid), dim3(RT), 0, s, n, 2, rh, r, r, r, xpart);
     HFX_HIP(hipGetLastError());
+    reduce(red.grid, 2, xpart, sc + SC_XSUMS);
     ++info.restarts;
     // Iterations up to the next restart.  The recurrence residual is checked
     // every check_every iterations; one iteration is queued behind each check
@@ -896,7 +939,7 @@ void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, con
         ++it;
       }
       if (it % check_every != 0 && it < o.maxits) continue;
-      hipLaunchKernelGGL(bicg_check_kernel, dim3(1), dim3(RT), 0, s, nx, xpart, target, ++seq, sc, st);
+      hipLaunchKernelGGL(bicg_check_kernel, dim3(1), dim3(RT), 0, s, np, xsums, target, ++seq, sc, st);
       HFX_HIP(hipGetLastError());
       if (caller_ws) {
         HFX_HIP(hipMemcpyAsync(&code, &st->code, sizeof(int), hipMemcpyDeviceToHost, s));
