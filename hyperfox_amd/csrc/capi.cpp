@@ -612,7 +612,7 @@ void do_solve(hfx_hdg* h, int pc, double rtol, int maxits, int restart, hfx::Kry
   o.restart = restart;
   o.graph = h->solver_graphs;
   if (h->krylov == HFX_KRYLOV_BICGSTAB) hfx::bicgstab(h->A, h->rhs.p, h->lambda.p, M, o, info, s, &h->kws);
-  else hfx::fgmres(h->A, h->rhs.p, h->lambda.p, M, o, info, s);
+  else hfx::fgmres(h->A, h->rhs.p, h->lambda.p, M, o, info, s, &h->kws);
 }
 
 }  // namespace

@@ -219,7 +219,7 @@ void solve(hfx_burgers* h, int pc, double rtol, int maxits, int restart, hfx::Kr
   o.restart = restart;
   o.graph = h->graphs;
   if (h->krylov == HFX_KRYLOV_BICGSTAB) hfx::bicgstab(h->A, h->rhs.p, h->trace.p, M, o, info, s, &h->kws);
-  else hfx::fgmres(h->A, h->rhs.p, h->trace.p, M, o, info, s);
+  else hfx::fgmres(h->A, h->rhs.p, h->trace.p, M, o, info, s, &h->kws);
   const int mu = m.nN * h->m;
   hfx::launch_reconstruct(m.nCells, mu, mu * h->dim, m.nFpc, h->bs(), h->U.p, h->U0.p, h->Q.p, h->Q0.p, h->c2f.p,
                           h->perm_m.p, h->trace.p, h->sol.p, h->flux.p, s);

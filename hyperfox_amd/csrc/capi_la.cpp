@@ -372,7 +372,7 @@ extern "C" int hfx_la_solve(hfx_la* h, double* x, int n, int* info, double* relr
     o.maxits = h->maxits;
     o.restart = h->restart;
     if (h->solver == HFX_LA_BCGS) hfx::bicgstab(h->A, h->db.p, h->dx.p, M, o, ki, s, &h->kws);
-    else hfx::fgmres(h->A, h->db.p, h->dx.p, M, o, ki, s);
+    else hfx::fgmres(h->A, h->db.p, h->dx.p, M, o, ki, s, &h->kws);
     h->dx.download(x, h->n, s);
     HFX_HIP(hipStreamSynchronize(s));
   }

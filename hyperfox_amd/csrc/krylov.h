@@ -97,16 +97,14 @@ struct Reducer {
   void init(long long n, double* mem);
   // out[j] = V_j . w for j < k (V column-major, leading dim ldv); result on device in out.p
   void multidot(long long n, int k, const double* V, long long ldv, const double* w, hipStream_t s);
-  // w -= sum_j h[j] V_j ; then out[k] = ||w||^2 partial-reduced (device h, k <= 64)
-  void update_norm(long long n, int k, const double* V, long long ldv, const double* h, double* w, double* out_norm2,
-                   hipStream_t s);
   double norm(long long n, const double* x, hipStream_t s);  // synchronous
 };
 
-// Right-preconditioned flexible GMRES(restart).  x holds the initial guess on
-// entry.
+// Right-preconditioned flexible GMRES(restart), classical Gram-Schmidt with one
+// re-orthogonalisation, Hessenberg matrix and stopping test on the device.  x
+// holds the initial guess on entry.
 void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
-            hipStream_t s);
+            hipStream_t s, KrylovWs* kws);
 
 // Right-preconditioned BiCGStab with device-resident scalars (no host round
 // trip per iteration; the recurrence residual is checked every 8 iterations).

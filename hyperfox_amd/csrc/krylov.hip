@@ -186,48 +186,6 @@ __global__ void reduce_rows_kernel(int G, const double* __restrict__ partial, do
   if (threadIdx.x == 0) out[j] = s;
 }
 
-__global__ void update_norm_kernel(long long n, int k, const double* __restrict__ V, long long ldv,
-                                   const double* __restrict__ h, double* __restrict__ w, double* __restrict__ partial) {
-  __shared__ double red[RT / 64];
-  __shared__ double hs[64];
-  if (threadIdx.x < k) hs[threadIdx.x] = h[threadIdx.x];
-  __syncthreads();
-  const int G = gridDim.x;
-  double acc = 0.0;
-  for (long long i = (long long)blockIdx.x * RT + threadIdx.x; i < n; i += (long long)G * RT) {
-    double wi = w[i];
-    for (int j = 0; j < k; ++j) wi -= hs[j] * V[(size_t)j * ldv + i];
-    w[i] = wi;
-    acc += wi * wi;
-  }
-  double s = block_sum(acc, red);
-  if (threadIdx.x == 0) partial[blockIdx.x] = s;
-}
-
-__global__ void scale_by_inv_sqrt_kernel(long long n, const double* __restrict__ norm2, const double* __restrict__ w,
-                                         double* __restrict__ v) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const double nv = sqrt(*norm2);
-  if (t < n) v[t] = nv > 0.0 ? w[t] / nv : 0.0;
-}
-
-__global__ void scale_kernel(long long n, double a, const double* __restrict__ x, double* __restrict__ y) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) y[t] = a * x[t];
-}
-
-// x += sum_j y_j Z_j
-__global__ void combine_kernel(long long n, int k, const double* __restrict__ Z, long long ldz,
-                               const double* __restrict__ y, double* __restrict__ x) {
-  __shared__ double ys[64];
-  if (threadIdx.x < k) ys[threadIdx.x] = y[threadIdx.x];
-  __syncthreads();
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  double acc = x[t];
-  for (int j = 0; j < k; ++j) acc += ys[j] * Z[(size_t)j * ldz + t];
-  x[t] = acc;
-}
 
 
 // ---------------------------------------------------------------- BiCGStab
@@ -511,6 +469,297 @@ __global__ void set_scalars_kernel(double* __restrict__ sc) {
   if (threadIdx.x < SC_N) sc[threadIdx.x] = 0.0;
 }
 
+// ------------------------------------------------------------------ GMRES
+//
+// One Arnoldi step is four launches (and the preconditioner's own, where it is
+// not fused): normalise v_j and apply M; w = A z with the products V^T w; one
+// pass that subtracts V h and forms V^T w again (the re-orthogonalisation); one
+// that subtracts the second h and forms the norm.  V is read three times.  The
+// Hessenberg column, its Givens rotations and the stopping test run on the
+// device, in a spare block of the next step's product, so the host only limits
+// how far it runs ahead.  Once the test has set the done flag every later
+// kernel returns at once.  The flag changes while a product kernel runs, so the
+// product reads a copy that the v kernel before it makes.
+//
+// State gs (doubles): cs, sn, g, h1, h2, y (64 or 65 each), R (column c at
+// c * 64), the last norm^2 and three ints: done, columns finished, the copy.
+enum { GM_CS = 0, GM_SN = 64, GM_G = 128, GM_H1 = 196, GM_H2 = 260, GM_Y = 324, GM_NORM2 = 388, GM_FLAGS = 390,
+       GM_R = 392, GM_N = 392 + 64 * 64 };
+enum { GM_DONE = 0, GM_COLS = 1, GM_SEEN = 2 };  // ints at gs + GM_FLAGS
+
+__device__ __forceinline__ int gm_flag(const double* gs, int which) {
+  return reinterpret_cast<const int*>(gs + GM_FLAGS)[which];
+}
+
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+  return __hiloint2double(hi, lo);
+}
+
+// Finish column c of the Hessenberg matrix (h1 + h2 and the norm): apply the
+// earlier rotations, make the new one, test for convergence.  One wavefront,
+// row i of the column in lane i.
+__device__ inline void gm_column(int c, double norm2, double target, int seq, double* gs, KrylovStatus* st) {
+  const int lane = threadIdx.x;
+  double h = lane <= c ? gs[GM_H1 + lane] + gs[GM_H2 + lane] : 0.0;
+  const double cs = gs[GM_CS + lane], sn = gs[GM_SN + lane];
+  const double hn = sqrt(norm2);
+  double t = lane_value(h, 0);
+  for (int i = 0; i < c; ++i) {
+    const double a1 = lane_value(h, i + 1), ci = lane_value(cs, i), si = lane_value(sn, i);
+    const double ri = ci * t + si * a1;
+    t = -si * t + ci * a1;
+    if (lane == i) h = ri;
+  }
+  const double rr = hypot(t, hn);
+  const double cc = rr != 0.0 ? t / rr : 1.0, sc = rr != 0.0 ? hn / rr : 0.0;
+  if (lane == c) h = rr;
+  if (lane <= c) gs[GM_R + c * 64 + lane] = h;
+  if (lane == 0) {
+    const double g = gs[GM_G + c], g1 = -sc * g;
+    gs[GM_CS + c] = cc;
+    gs[GM_SN + c] = sc;
+    gs[GM_G + c] = cc * g;
+    gs[GM_G + c + 1] = g1;
+    const int done = !isfinite(g1) || fabs(g1) <= target || hn == 0.0;
+    int* f = reinterpret_cast<int*>(gs + GM_FLAGS);
+    f[GM_DONE] = done;
+    f[GM_COLS] = c + 1;
+    __hip_atomic_store(&st->code, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&st->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+__global__ void gm_start_kernel(double beta, double* __restrict__ gs) {
+  for (int i = threadIdx.x; i < GM_R; i += blockDim.x) gs[i] = i == GM_G ? beta : 0.0;
+}
+
+// v_j = w / ||w|| (||w||^2 from part; j = 0: r / beta), z = M v_j
+template <int PC, int BS>
+__global__ __launch_bounds__(RT) void gm_v_kernel(long long n, int j, double ibeta, int np,
+                                                  const double* __restrict__ part, const double* __restrict__ w,
+                                                  const double* __restrict__ dinv, double* __restrict__ v,
+                                                  double* __restrict__ z, double* __restrict__ gs) {
+  __shared__ double red[2][SV / 64];
+  __shared__ double xs[PC == PC_BJACOBI ? RT : 1];
+  if (gm_flag(gs, GM_DONE)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) reinterpret_cast<int*>(gs + GM_FLAGS)[GM_SEEN] = 1;
+    return;
+  }
+  constexpr int TR = tile_rows<PC, BS>();
+  const long long t = (long long)blockIdx.x * TR + threadIdx.x;
+  const bool on = threadIdx.x < TR && t < n;
+  double x = on ? w[t] : 0.0;
+  if (j == 0) {
+    x *= ibeta;
+  } else {
+    double norm2, unused;
+    partial_sums(np, part, false, norm2, unused, red);
+    const double nv = sqrt(norm2);
+    x = nv > 0.0 ? x / nv : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) gs[GM_NORM2] = norm2;
+  }
+  if (on) v[t] = x;
+  apply_tile<PC, BS>(on, t, x, dinv, z, xs);
+}
+
+// Sums over the wavefront of KC values per lane at once: each step halves the
+// values a lane holds and exchanges the other half (KC - 1 exchanges for all
+// of them, against 6 KC for KC separate trees).  The sum of value
+// sum_index<KC>(lane) ends in every lane of its group.
+template <int KC>
+__device__ __forceinline__ double wave_sums(double* v) {
+  const int lane = threadIdx.x & 63;
+  int m = 32;
+#pragma unroll
+  for (int K = KC / 2; K >= 1; K >>= 1, m >>= 1) {
+    const bool up = (lane & m) != 0;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const double keep = up ? v[i + K] : v[i], send = up ? v[i] : v[i + K];
+      v[i] = keep + __shfl_xor(send, m, 64);
+    }
+  }
+  double s = v[0];
+  for (; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
+  return s;
+}
+template <int KC>
+__device__ __forceinline__ int sum_index(int lane) {
+  int idx = 0, m = 32;
+#pragma unroll
+  for (int K = KC / 2; K >= 1; K >>= 1, m >>= 1) idx += (lane & m) ? K : 0;
+  return idx;
+}
+
+// partial[(c0 + i) nblk + blk] = sum over the block of v[i], c0 + i < k
+template <int KC>
+__device__ __forceinline__ void block_sums(double* v, int c0, int k, double* __restrict__ partial, int nblk, int blk,
+                                           double (*red)[KC]) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const double s = wave_sums<KC>(v);
+  __syncthreads();  // red is free
+  if ((lane & (64 / KC - 1)) == 0) red[wid][sum_index<KC>(lane)] = s;
+  __syncthreads();
+  if (threadIdx.x < KC && c0 + threadIdx.x < k) {
+    double a = 0.0;
+#pragma unroll
+    for (int q = 0; q < RT / 64; ++q) a += red[q][threadIdx.x];
+    partial[(size_t)(c0 + threadIdx.x) * nblk + blk] = a;
+  }
+}
+
+// w = A z (thread per row) with the partials of V_i . w, i < k, in
+// partial[i nblk + blk]; block nblk finishes Hessenberg column k - 2.
+template <int BS, int KC>
+__global__ __launch_bounds__(RT) void gm_product_kernel(int nb, const int* __restrict__ rowptr,
+                                                        const int* __restrict__ col, const double* __restrict__ vals,
+                                                        const double* __restrict__ z, double* __restrict__ w, int k,
+                                                        const double* __restrict__ V, long long ldv, int nblk,
+                                                        double* __restrict__ partial, double target, int seq,
+                                                        double* gs, KrylovStatus* st) {
+  __shared__ double red[RT / 64][KC];
+  if (gm_flag(gs, GM_SEEN)) return;
+  if ((int)blockIdx.x == nblk) {
+    if (threadIdx.x < 64) gm_column(k - 2, gs[GM_NORM2], target, seq, gs, st);
+    return;
+  }
+  const long long t = (long long)blockIdx.x * RT + threadIdx.x;
+  const bool on = t < (long long)nb * BS;
+  double acc = 0.0;
+  if (on) {
+    const int F = (int)(t / BS), r = (int)(t % BS);
+    acc = bsr_row_sum<BS>(rowptr[F], rowptr[F + 1], r, nullptr, col, vals, z);
+    w[t] = acc;
+  }
+  for (int c0 = 0; c0 < k; c0 += KC) {
+    double v[KC];
+#pragma unroll
+    for (int i = 0; i < KC; ++i) v[i] = on && c0 + i < k ? V[(size_t)(c0 + i) * ldv + t] * acc : 0.0;
+    block_sums<KC>(v, c0, k, partial, nblk, blockIdx.x, red);
+  }
+}
+
+// h[i] = sum of the np partials of row i, i < k, in LDS (np = 1: already
+// reduced); block 0 keeps them for the Hessenberg column
+__device__ __forceinline__ void gather_h(int k, int np, const double* __restrict__ part, double* hs,
+                                         double* __restrict__ keep) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (np == 1) {
+    if (threadIdx.x < k) hs[threadIdx.x] = part[threadIdx.x];
+  } else {
+    for (int i0 = wid * 4; i0 < k; i0 += RT / 64 * 4) {
+      double a[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a[u] = 0.0;
+        if (i0 + u < k)
+          for (int b = lane; b < np; b += 64) a[u] += part[(size_t)(i0 + u) * np + b];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a[u] = wave_sum(a[u]);
+        if (lane == 0 && i0 + u < k) hs[i0 + u] = a[u];
+      }
+    }
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && threadIdx.x < k) keep[threadIdx.x] = hs[threadIdx.x];
+}
+
+// w -= V h, then the partials of V_i . w: the V values of a row stay in
+// registers between the two (up to KC of them)
+template <int KC>
+__global__ __launch_bounds__(RT) void gm_orth_kernel(long long n, int k, const double* __restrict__ V, long long ldv,
+                                                     int np, const double* __restrict__ part, double* __restrict__ w,
+                                                     int nblk, double* __restrict__ partial, double* gs) {
+  __shared__ double hs[64];
+  __shared__ double red[RT / 64][KC];
+  if (gm_flag(gs, GM_DONE)) return;
+  const long long t = (long long)blockIdx.x * RT + threadIdx.x;
+  const bool on = t < n;
+  double x = on ? w[t] : 0.0;
+  double v[KC];
+#pragma unroll
+  for (int i = 0; i < KC; ++i) v[i] = on && i < k ? V[(size_t)i * ldv + t] : 0.0;
+  gather_h(k, np, part, hs, gs + GM_H1);
+#pragma unroll
+  for (int i = 0; i < KC; ++i)
+    if (i < k) x -= hs[i] * v[i];
+  for (int i = KC; i < k; ++i) x -= hs[i] * (on ? V[(size_t)i * ldv + t] : 0.0);
+  if (on) w[t] = x;
+  for (int c0 = 0; c0 < k; c0 += KC) {
+#pragma unroll
+    for (int i = 0; i < KC; ++i) {
+      if (c0 > 0) v[i] = on && c0 + i < k ? V[(size_t)(c0 + i) * ldv + t] : 0.0;
+      v[i] *= x;
+    }
+    block_sums<KC>(v, c0, k, partial, nblk, blockIdx.x, red);
+  }
+}
+
+// w -= V h, with the partials of w . w
+__global__ __launch_bounds__(RT) void gm_norm_kernel(long long n, int k, const double* __restrict__ V, long long ldv,
+                                                     int np, const double* __restrict__ part, double* __restrict__ w,
+                                                     double* __restrict__ partial, double* gs) {
+  __shared__ double hs[64];
+  __shared__ double red[RT / 64];
+  if (gm_flag(gs, GM_DONE)) return;
+  const long long t = (long long)blockIdx.x * RT + threadIdx.x;
+  const bool on = t < n;
+  double x = on ? w[t] : 0.0;
+  gather_h(k, np, part, hs, gs + GM_H2);
+  if (on) {
+#pragma unroll 8
+    for (int i = 0; i < k; ++i) x -= hs[i] * V[(size_t)i * ldv + t];
+    w[t] = x;
+  }
+  const double s = block_sum(x * x, red);
+  if (threadIdx.x == 0) partial[blockIdx.x] = s;
+}
+
+// End of a cycle: finish the last column (c, when the done flag has not cut
+// the cycle short), then back substitution R y = g
+__global__ __launch_bounds__(RT) void gm_finish_kernel(int c, int np, const double* __restrict__ part, double target,
+                                                       int seq, double* gs, KrylovStatus* st) {
+  __shared__ double red[2][SV / 64];
+  double norm2, unused;
+  partial_sums(np, part, false, norm2, unused, red);
+  if (threadIdx.x >= 64) return;
+  if (!gm_flag(gs, GM_DONE)) gm_column(c, norm2, target, seq - 1, gs, st);
+  __threadfence_block();
+  __builtin_amdgcn_wave_barrier();
+  const int lane = threadIdx.x, k = reinterpret_cast<const volatile int*>(gs + GM_FLAGS)[GM_COLS];
+  double g = lane < k ? gs[GM_G + lane] : 0.0, y = 0.0;
+  for (int i = k - 1; i >= 0; --i) {
+    const double ri = lane <= i ? gs[GM_R + i * 64 + lane] : 0.0;
+    const double d = lane_value(ri, i), yi = d != 0.0 ? lane_value(g, i) / d : 0.0;
+    if (lane == i) y = yi;
+    if (lane < i) g -= ri * yi;
+  }
+  gs[GM_Y + lane] = y;
+  if (lane == 0) {
+    __hip_atomic_store(&st->code, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&st->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// x += sum_j y_j Z_j over the columns of the cycle
+__global__ __launch_bounds__(RT) void gm_combine_kernel(long long n, const double* __restrict__ Z, long long ldz,
+                                                        const double* __restrict__ gs, double* __restrict__ x) {
+  __shared__ double ys[64];
+  const int k = gm_flag(gs, GM_COLS);
+  if (threadIdx.x < 64) ys[threadIdx.x] = gs[GM_Y + threadIdx.x];
+  __syncthreads();
+  const long long t = (long long)blockIdx.x * RT + threadIdx.x;
+  if (t >= n) return;
+  double acc = x[t];
+#pragma unroll 8
+  for (int j = 0; j < k; ++j) acc += ys[j] * Z[(size_t)j * ldz + t];
+  x[t] = acc;
+}
+
 }  // namespace
 
 void bsr_spmv(const BsrDev& A, const double* x, double* y, const double* b, hipStream_t s) {
@@ -605,15 +854,6 @@ void Reducer::multidot(long long n, int k, const double* V, long long ldv, const
   HFX_HIP(hipGetLastError());
 }
 
-void Reducer::update_norm(long long n, int k, const double* V, long long ldv, const double* h, double* w,
-                          double* out_norm2, hipStream_t s) {
-  if (k > 64) throw std::runtime_error("update: at most 64 vectors");
-  hipLaunchKernelGGL(update_norm_kernel, dim3(grid), dim3(RT), 0, s, n, k, V, ldv, h, w, partial);
-  HFX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(reduce_rows_kernel, dim3(1), dim3(RT), 0, s, grid, partial, out_norm2);
-  HFX_HIP(hipGetLastError());
-}
-
 double Reducer::norm(long long n, const double* x, hipStream_t s) {
   multidot(n, 1, x, 0, x, s);
   double v = 0.0;
@@ -621,103 +861,6 @@ double Reducer::norm(long long n, const double* x, hipStream_t s) {
   HFX_HIP(hipStreamSynchronize(s));
   return std::sqrt(v);
 }
-
-void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
-            hipStream_t s) {
-  const long long n = A.nrows();
-  const int m = o.restart;
-  if (m < 1 || m > 63) throw std::runtime_error("gmres: restart must be in [1, 63]");
-  info = KrylovInfo();
-  Reducer red;
-  red.init(n);
-  DevBuf<double> V, Zb, w, r, hdev;
-  V.alloc((size_t)(m + 1) * n);
-  Zb.alloc((size_t)m * n);
-  w.alloc(n);
-  r.alloc(n);
-  hdev.alloc(2 * 64 + 4);
-  const double bnorm = red.norm(n, b, s);
-  if (bnorm == 0.0) {
-    HFX_HIP(hipMemsetAsync(x, 0, n * sizeof(double), s));
-    HFX_HIP(hipStreamSynchronize(s));
-    info.reason = CONVERGED_ATOL;
-    return;
-  }
-  const double target = o.rtol * bnorm;
-  std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), y(m), hh(2 * 64 + 2);
-  int it = 0;
-  while (true) {
-    bsr_spmv(A, x, r.p, b, s);  // r = b - A x (true FP64 residual)
-    const double beta = red.norm(n, r.p, s);
-    info.true_relres = beta / bnorm;
-    if (!std::isfinite(beta)) { info.reason = DIVERGED_NANORINF; break; }
-    if (beta <= target) { info.reason = CONVERGED_RTOL; break; }
-    if (it >= o.maxits) { info.reason = DIVERGED_ITS; break; }
-    hipLaunchKernelGGL(scale_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, n, 1.0 / beta, r.p, V.p);
-    HFX_HIP(hipGetLastError());
-    std::fill(g.begin(), g.end(), 0.0);
-    g[0] = beta;
-    int k = 0;
-    bool done = false;
-    for (; k < m && it < o.maxits; ++k) {
-      double* vk = V.p + (size_t)k * n;
-      double* zk = Zb.p + (size_t)k * n;
-      if (M.kind != PC_NONE) M.fn(vk, zk);
-      else HFX_HIP(hipMemcpyAsync(zk, vk, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-      bsr_spmv(A, zk, w.p, nullptr, s);
-      // classical Gram-Schmidt, twice
-      red.multidot(n, k + 1, V.p, n, w.p, s);
-      HFX_HIP(hipMemcpyAsync(hdev.p, red.out, (k + 1) * sizeof(double), hipMemcpyDeviceToDevice, s));
-      red.update_norm(n, k + 1, V.p, n, hdev.p, w.p, hdev.p + 128, s);
-      red.multidot(n, k + 1, V.p, n, w.p, s);
-      HFX_HIP(hipMemcpyAsync(hdev.p + 64, red.out, (k + 1) * sizeof(double), hipMemcpyDeviceToDevice, s));
-      red.update_norm(n, k + 1, V.p, n, hdev.p + 64, w.p, hdev.p + 128, s);
-      hipLaunchKernelGGL(scale_by_inv_sqrt_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, n, hdev.p + 128, w.p,
-                         V.p + (size_t)(k + 1) * n);
-      HFX_HIP(hipGetLastError());
-      HFX_HIP(hipMemcpyAsync(hh.data(), hdev.p, (2 * 64 + 1) * sizeof(double), hipMemcpyDeviceToHost, s));
-      HFX_HIP(hipStreamSynchronize(s));
-      ++it;
-      for (int j = 0; j <= k; ++j) H[(size_t)j * m + k] = hh[j] + hh[64 + j];
-      const double hn = std::sqrt(hh[128]);
-      H[(size_t)(k + 1) * m + k] = hn;
-      for (int j = 0; j < k; ++j) {
-        const double a0 = H[(size_t)j * m + k], a1 = H[(size_t)(j + 1) * m + k];
-        H[(size_t)j * m + k] = cs[j] * a0 + sn[j] * a1;
-        H[(size_t)(j + 1) * m + k] = -sn[j] * a0 + cs[j] * a1;
-      }
-      const double a0 = H[(size_t)k * m + k], a1 = H[(size_t)(k + 1) * m + k];
-      const double rr = std::hypot(a0, a1);
-      cs[k] = rr != 0.0 ? a0 / rr : 1.0;
-      sn[k] = rr != 0.0 ? a1 / rr : 0.0;
-      H[(size_t)k * m + k] = rr;
-      H[(size_t)(k + 1) * m + k] = 0.0;
-      g[k + 1] = -sn[k] * g[k];
-      g[k] = cs[k] * g[k];
-      if (!std::isfinite(g[k + 1])) { done = true; ++k; break; }
-      if (std::fabs(g[k + 1]) <= target || hn == 0.0) { done = true; ++k; break; }
-    }
-    // solve the k x k triangular system and update x += Z y
-    for (int i = k - 1; i >= 0; --i) {
-      double acc = g[i];
-      for (int j = i + 1; j < k; ++j) acc -= H[(size_t)i * m + j] * y[j];
-      y[i] = H[(size_t)i * m + i] != 0.0 ? acc / H[(size_t)i * m + i] : 0.0;
-    }
-    if (k > 0) {
-      HFX_HIP(hipMemcpyAsync(hdev.p, y.data(), k * sizeof(double), hipMemcpyHostToDevice, s));
-      hipLaunchKernelGGL(combine_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, n, k, Zb.p, n, hdev.p, x);
-      HFX_HIP(hipGetLastError());
-    }
-    ++info.restarts;
-    (void)done;
-  }
-  info.iters = it;
-  HFX_HIP(hipStreamSynchronize(s));
-}
-
-}  // namespace hfx
-
-namespace hfx {
 
 KrylovWs::~KrylovWs() {
   if (status) (void)hipHostFree(status);
@@ -751,11 +894,6 @@ void KrylovWs::wait(int seq, hipStream_t s) const {
   }
 }
 
-size_t bicgstab_ws_doubles(long long n) {
-  const size_t G = (size_t)Reducer::grid_for(n), nblk_rows = (size_t)ceil_div(n, RT);
-  return al32(Reducer::doubles(n)) + 8 * al32((size_t)n) + al32(SC_N) + al32(2 * G) + al32(2 * nblk_rows);
-}
-
 // Vectors of up to this many 256-row blocks have their dot products' partials
 // added up again by every block of the next kernel; beyond it a one-block
 // kernel reduces them first.  At the line each of the (at most 2048) blocks
@@ -763,6 +901,150 @@ size_t bicgstab_ws_doubles(long long n) {
 // (3.8 us + 2 us of gap on systems of 40,000 to 300,000 rows, where BiCGStab
 // is bound by its launches).
 constexpr int INLINE_PARTIALS = 2048;
+
+// Steps whose vectors span at most this many 256-row blocks leave the partials
+// of V^T w for every block of the next kernel to add up (k x 128 values out of
+// L2, about the time of the extra launch); longer ones reduce them first.
+constexpr int GM_INLINE = 128;
+
+void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
+            hipStream_t s, KrylovWs* kws) {
+  const long long n = A.nrows();
+  const int m = o.restart;
+  if (m < 1 || m > 63) throw std::runtime_error("gmres: restart must be in [1, 63]");
+  info = KrylovInfo();
+  const int nblk = ceil_div(n, RT);
+  // V (m + 1), Z (m), w, r, the partials of two V^T w and of a norm, the state
+  DevBuf<double> own;
+  const size_t ln = al32((size_t)n);
+  const size_t need = al32(Reducer::doubles(n)) + (size_t)(2 * m + 3) * ln + 2 * al32((size_t)64 * nblk) +
+                      al32((size_t)nblk) + al32(GM_N) + al32(128);
+  KrylovWs local;
+  KrylovWs& hw = kws ? *kws : local;
+  double* ws = hw.mem_for(need, own);
+  Reducer red;
+  red.init(n, ws);
+  double* q = ws + al32(Reducer::doubles(n));
+  auto take = [&q](size_t k) { double* r0 = q; q += al32(k); return r0; };
+  double* V = take((size_t)(m + 1) * ln);
+  double* Z = take((size_t)m * ln);
+  double *w = take(n), *r = take(n);
+  double *p1 = take((size_t)64 * nblk), *p2 = take((size_t)64 * nblk), *p3 = take(nblk);
+  double* gs = take(GM_N);
+  double* hr = take(128);  // reduced h1, h2
+  const double bnorm = red.norm(n, b, s);
+  if (bnorm == 0.0) {
+    HFX_HIP(hipMemsetAsync(x, 0, n * sizeof(double), s));
+    HFX_HIP(hipStreamSynchronize(s));
+    info.reason = CONVERGED_ATOL;
+    return;
+  }
+  const double target = o.rtol * bnorm;
+  KrylovStatus* st = hw.host();
+  const bool inl = nblk <= GM_INLINE, inl3 = nblk <= INLINE_PARTIALS;
+  const int tiles = M.kind == PC_BJACOBI ? ceil_div(n, (RT / A.bs) * A.bs) : nblk;
+  double* sums3 = inl3 ? p3 : gs + GM_NORM2 + 1;  // ||w||^2
+  const int np3 = inl3 ? nblk : 1;
+  auto vstep = [&](int j, double ibeta) {
+    const double* src = j == 0 ? r : w;
+    double *v = V + (size_t)j * ln, *z = Z + (size_t)j * ln;
+#define HFX_LAUNCH(PC, B)                                                                                          \
+  hipLaunchKernelGGL((gm_v_kernel<PC, B>), dim3(tiles), dim3(RT), 0, s, n, j, ibeta, np3, sums3, src, M.dinv, v, z, gs)
+#define HFX_BS(B) case B: HFX_LAUNCH(PC_BJACOBI, B); break;
+    if (M.kind == PC_NONE) HFX_LAUNCH(PC_NONE, 1);
+    else if (M.kind == PC_JACOBI) HFX_LAUNCH(PC_JACOBI, 1);
+    else if (M.kind == PC_OTHER) HFX_LAUNCH(PC_OTHER, 1);
+    else switch (A.bs) {
+      HFX_BS(1) HFX_BS(2) HFX_BS(3) HFX_BS(4) HFX_BS(5) HFX_BS(6) HFX_BS(7) HFX_BS(8) HFX_BS(9) HFX_BS(10) HFX_BS(11) HFX_BS(12) HFX_BS(15) HFX_BS(18) HFX_BS(21) HFX_BS(30)
+      default: throw std::runtime_error("gmres: unsupported block size");
+    }
+#undef HFX_BS
+#undef HFX_LAUNCH
+    HFX_HIP(hipGetLastError());
+    if (M.kind == PC_OTHER) M.fn(v, z);
+  };
+  auto product = [&](int j, int seq) {
+    const int k = j + 1, grid = nblk + (j > 0 ? 1 : 0);
+    const double* z = Z + (size_t)j * ln;
+#define HFX_LAUNCH(B, KC)                                                                                           \
+  hipLaunchKernelGGL((gm_product_kernel<B, KC>), dim3(grid), dim3(RT), 0, s, A.nb, A.rowptr.p, A.col.p, A.vals.p, z, \
+                     w, k, V, (long long)ln, nblk, p1, target, seq, gs, st)
+#define HFX_BS(B) case B: if (k <= 8) HFX_LAUNCH(B, 8); else HFX_LAUNCH(B, 32); break;
+    switch (A.bs) {
+      HFX_BS(1) HFX_BS(2) HFX_BS(3) HFX_BS(4) HFX_BS(5) HFX_BS(6) HFX_BS(7) HFX_BS(8) HFX_BS(9) HFX_BS(10) HFX_BS(11) HFX_BS(12) HFX_BS(15) HFX_BS(18) HFX_BS(21) HFX_BS(30)
+      default: throw std::runtime_error("spmv: unsupported block size");
+    }
+#undef HFX_BS
+#undef HFX_LAUNCH
+    HFX_HIP(hipGetLastError());
+  };
+  // the partials of V^T w, or (long vectors) their sums
+  auto rows = [&](int k, const double* part, double* sums) -> const double* {
+    if (inl) return part;
+    hipLaunchKernelGGL(reduce_rows_kernel, dim3(k), dim3(RT), 0, s, nblk, part, sums);
+    HFX_HIP(hipGetLastError());
+    return sums;
+  };
+  const int nph = inl ? nblk : 1;
+  int it = 0, base = 0;
+  while (true) {
+    bsr_spmv(A, x, r, b, s);  // r = b - A x (true FP64 residual)
+    const double beta = red.norm(n, r, s);
+    info.true_relres = beta / bnorm;
+    if (!std::isfinite(beta)) { info.reason = DIVERGED_NANORINF; break; }
+    if (beta <= target) { info.reason = CONVERGED_RTOL; break; }
+    if (it >= o.maxits) { info.reason = DIVERGED_ITS; break; }
+    hipLaunchKernelGGL(gm_start_kernel, dim3(1), dim3(256), 0, s, beta, gs);
+    HFX_HIP(hipGetLastError());
+    int j = 0;
+    for (; j < m && it + j < o.maxits; ++j) {
+      // column j - 4 has been tested before step j is queued: at most three
+      // steps run past the end of a cycle, as kernels that return at once
+      if (j >= 4) {
+        hw.wait(base + j - 3, s);
+        if (__atomic_load_n(&st->code, __ATOMIC_RELAXED) != 0) break;
+      }
+      const int k = j + 1;
+      vstep(j, 1.0 / beta);
+      product(j, base + j);
+      const double* h1 = rows(k, p1, hr);
+      if (k <= 8)
+        hipLaunchKernelGGL((gm_orth_kernel<8>), dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h1, w, nblk,
+                           p2, gs);
+      else
+        hipLaunchKernelGGL((gm_orth_kernel<32>), dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h1, w, nblk,
+                           p2, gs);
+      HFX_HIP(hipGetLastError());
+      const double* h2 = rows(k, p2, hr + 64);
+      hipLaunchKernelGGL(gm_norm_kernel, dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h2, w, p3, gs);
+      HFX_HIP(hipGetLastError());
+      if (!inl3) {
+        hipLaunchKernelGGL(reduce_rows_kernel, dim3(1), dim3(RT), 0, s, nblk, p3, sums3);
+        HFX_HIP(hipGetLastError());
+      }
+    }
+    // column j - 1 is still open unless the done flag was set by then
+    hipLaunchKernelGGL(gm_finish_kernel, dim3(1), dim3(RT), 0, s, j - 1, np3, sums3, target, base + 100, gs, st);
+    HFX_HIP(hipGetLastError());
+    hipLaunchKernelGGL(gm_combine_kernel, dim3(nblk), dim3(RT), 0, s, n, Z, (long long)ln, gs, x);
+    HFX_HIP(hipGetLastError());
+    hw.wait(base + 100, s);
+    it += __atomic_load_n(&st->code, __ATOMIC_RELAXED);
+    base += 128;
+    ++info.restarts;
+  }
+  info.iters = it;
+  HFX_HIP(hipStreamSynchronize(s));
+}
+
+}  // namespace hfx
+
+namespace hfx {
+
+size_t bicgstab_ws_doubles(long long n) {
+  const size_t G = (size_t)Reducer::grid_for(n), nblk_rows = (size_t)ceil_div(n, RT);
+  return al32(Reducer::doubles(n)) + 8 * al32((size_t)n) + al32(SC_N) + al32(2 * G) + al32(2 * nblk_rows);
+}
 
 void bicgstab(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
               hipStream_t s, KrylovWs* kws, double* ws) {

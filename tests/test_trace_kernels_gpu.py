@@ -74,3 +74,38 @@ def test_reconstruction(dim, p, n):
         ref = np.einsum('eij,ej->ei', M, lc) + M0
         mag = np.einsum('eij,ej->ei', np.abs(M), np.abs(lc)) + np.abs(M0)
         assert (np.abs(got - ref) <= 2 * (lc.shape[1] + 1) * EPS * mag).all()
+
+
+@pytest.mark.parametrize('restart', [1, 2, 8, 9, 31, 33, 63])
+@pytest.mark.parametrize('n', [1, 7, 19])
+def test_gmres_against_a_dense_solve(n, restart):
+    """Restart lengths around the register tiles (8 and 32 columns), one and several row blocks, an iteration budget
+    inside a cycle, and convergence inside a cycle.  At rtol the residual is at most rtol ||b||, so the error is at
+    most cond(A) rtol ||x||."""
+    print('gmres', n, restart, flush=True)
+    rng = np.random.default_rng(n)
+    N = n * n + 3
+    A = 4.0 * np.eye(N) + 0.5 * (np.eye(N, k=1) + np.eye(N, k=-1)) + 0.2 * np.eye(N, k=3)
+    A += np.diag(rng.random(N))
+    b = rng.standard_normal(N)
+    la = hf.HipLinAlgebra(hf.HipOpts(rtol=1e-11, maxits=2000, restart=restart))
+    la.initialize()
+    la.configure()
+    la.allocate(N)
+    for i in range(N):
+        cols = np.nonzero(A[i])[0]
+        la.setValsMatrix([i], cols, A[i, cols])
+    la.setValsRHS(np.arange(N), b)
+    la.assemble()
+    x = np.array(la.solve())
+    its, reason, rel = la.last_info
+    assert reason == 2 and rel <= 1e-11
+    ref = np.linalg.solve(A, b)
+    assert np.linalg.norm(x - ref) <= np.linalg.cond(A) * 1e-11 * np.linalg.norm(ref)
+    # a second solve of the same handle repeats the first bit for bit
+    assert np.array_equal(np.array(la.solve()), x) and la.last_info[0] == its
+    if its > 3:
+        la.options.maxits = its - 1
+        la.configure()
+        la.solve()
+        assert la.last_info[:2] == (its - 1, -3) and la.last_info[2] > 1e-11
