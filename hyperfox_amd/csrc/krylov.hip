@@ -593,6 +593,17 @@ __device__ __forceinline__ int sum_index(int lane) {
   return idx;
 }
 
+// v[i] = V_(c0 + i)[t], 0 from column k on: loads at clamped columns, so that
+// they issue back to back without branches
+template <int KC>
+__device__ __forceinline__ void load_rows(const double* __restrict__ V, long long ldv, int c0, int k, long long t,
+                                          double* v) {
+#pragma unroll
+  for (int i = 0; i < KC; ++i) v[i] = V[(size_t)min(c0 + i, k - 1) * ldv + t];
+#pragma unroll
+  for (int i = 0; i < KC; ++i) v[i] = c0 + i < k ? v[i] : 0.0;
+}
+
 // partial[(c0 + i) nblk + blk] = sum over the block of v[i], c0 + i < k
 template <int KC>
 __device__ __forceinline__ void block_sums(double* v, int c0, int k, double* __restrict__ partial, int nblk, int blk,
@@ -633,10 +644,12 @@ __global__ __launch_bounds__(RT) void gm_product_kernel(int nb, const int* __res
     acc = bsr_row_sum<BS>(rowptr[F], rowptr[F + 1], r, nullptr, col, vals, z);
     w[t] = acc;
   }
+  const long long tc = on ? t : 0;
   for (int c0 = 0; c0 < k; c0 += KC) {
     double v[KC];
+    load_rows<KC>(V, ldv, c0, k, tc, v);
 #pragma unroll
-    for (int i = 0; i < KC; ++i) v[i] = on && c0 + i < k ? V[(size_t)(c0 + i) * ldv + t] * acc : 0.0;
+    for (int i = 0; i < KC; ++i) v[i] *= acc;
     block_sums<KC>(v, c0, k, partial, nblk, blockIdx.x, red);
   }
 }
@@ -649,19 +662,22 @@ __device__ __forceinline__ void gather_h(int k, int np, const double* __restrict
   if (np == 1) {
     if (threadIdx.x < k) hs[threadIdx.x] = part[threadIdx.x];
   } else {
-    for (int i0 = wid * 4; i0 < k; i0 += RT / 64 * 4) {
-      double a[4];
+    constexpr int U = 8;  // rows per wavefront at a time, their loads in flight together
+    for (int i0 = wid * U; i0 < k; i0 += RT / 64 * U) {
+      double a[U];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        a[u] = 0.0;
-        if (i0 + u < k)
-          for (int b = lane; b < np; b += 64) a[u] += part[(size_t)(i0 + u) * np + b];
+      for (int u = 0; u < U; ++u) {
+        const double* row = part + (size_t)min(i0 + u, k - 1) * np;
+        a[u] = row[min(lane, np - 1)];
+        a[u] = lane < np ? a[u] : 0.0;
+        for (int b = lane + 64; b < np; b += 64) a[u] += row[b];
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        a[u] = wave_sum(a[u]);
-        if (lane == 0 && i0 + u < k) hs[i0 + u] = a[u];
-      }
+      for (int u = 0; u < U; ++u) a[u] = wave_sum(a[u]);
+      if (lane == 0)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (i0 + u < k) hs[i0 + u] = a[u];
     }
   }
   __syncthreads();
@@ -680,21 +696,19 @@ __global__ __launch_bounds__(RT) void gm_orth_kernel(long long n, int k, const d
   const long long t = (long long)blockIdx.x * RT + threadIdx.x;
   const bool on = t < n;
   double x = on ? w[t] : 0.0;
+  const long long tc = on ? t : 0;
   double v[KC];
-#pragma unroll
-  for (int i = 0; i < KC; ++i) v[i] = on && i < k ? V[(size_t)i * ldv + t] : 0.0;
+  load_rows<KC>(V, ldv, 0, k, tc, v);
   gather_h(k, np, part, hs, gs + GM_H1);
 #pragma unroll
-  for (int i = 0; i < KC; ++i)
-    if (i < k) x -= hs[i] * v[i];
-  for (int i = KC; i < k; ++i) x -= hs[i] * (on ? V[(size_t)i * ldv + t] : 0.0);
+  for (int i = 0; i < KC; ++i) x -= (i < k ? hs[i] : 0.0) * v[i];
+  for (int i = KC; i < k; ++i) x -= hs[i] * V[(size_t)i * ldv + tc];
+  if (!on) x = 0.0;
   if (on) w[t] = x;
   for (int c0 = 0; c0 < k; c0 += KC) {
+    if (c0 > 0) load_rows<KC>(V, ldv, c0, k, tc, v);
 #pragma unroll
-    for (int i = 0; i < KC; ++i) {
-      if (c0 > 0) v[i] = on && c0 + i < k ? V[(size_t)(c0 + i) * ldv + t] : 0.0;
-      v[i] *= x;
-    }
+    for (int i = 0; i < KC; ++i) v[i] *= x;
     block_sums<KC>(v, c0, k, partial, nblk, blockIdx.x, red);
   }
 }
@@ -969,7 +983,7 @@ void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const
 #define HFX_LAUNCH(B, KC)                                                                                           \
   hipLaunchKernelGGL((gm_product_kernel<B, KC>), dim3(grid), dim3(RT), 0, s, A.nb, A.rowptr.p, A.col.p, A.vals.p, z, \
                      w, k, V, (long long)ln, nblk, p1, target, seq, gs, st)
-#define HFX_BS(B) case B: if (k <= 8) HFX_LAUNCH(B, 8); else HFX_LAUNCH(B, 32); break;
+#define HFX_BS(B) case B: if (k <= 8) HFX_LAUNCH(B, 8); else if (k <= 16) HFX_LAUNCH(B, 16); else HFX_LAUNCH(B, 32); break;
     switch (A.bs) {
       HFX_BS(1) HFX_BS(2) HFX_BS(3) HFX_BS(4) HFX_BS(5) HFX_BS(6) HFX_BS(7) HFX_BS(8) HFX_BS(9) HFX_BS(10) HFX_BS(11) HFX_BS(12) HFX_BS(15) HFX_BS(18) HFX_BS(21) HFX_BS(30)
       default: throw std::runtime_error("spmv: unsupported block size");
@@ -1008,12 +1022,12 @@ void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const
       vstep(j, 1.0 / beta);
       product(j, base + j);
       const double* h1 = rows(k, p1, hr);
-      if (k <= 8)
-        hipLaunchKernelGGL((gm_orth_kernel<8>), dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h1, w, nblk,
-                           p2, gs);
-      else
-        hipLaunchKernelGGL((gm_orth_kernel<32>), dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h1, w, nblk,
-                           p2, gs);
+#define HFX_LAUNCH(KC)                                                                                              \
+  hipLaunchKernelGGL((gm_orth_kernel<KC>), dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h1, w, nblk, p2, gs)
+      if (k <= 8) HFX_LAUNCH(8);
+      else if (k <= 16) HFX_LAUNCH(16);
+      else HFX_LAUNCH(32);
+#undef HFX_LAUNCH
       HFX_HIP(hipGetLastError());
       const double* h2 = rows(k, p2, hr + 64);
       hipLaunchKernelGGL(gm_norm_kernel, dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h2, w, p3, gs);
