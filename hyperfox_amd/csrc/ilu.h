@@ -18,7 +18,12 @@ namespace hfx {
 struct Ilu {
   int nb = 0, bs = 0, ordering = -1;
   IluPlan plan;
-  DevBuf<int> rowptr, fwd_rows, bwd_rows, lptr, lpos, lcol, uptr, upos, ucol, dslot, pptr, pslot, ppos, err;
+  DevBuf<int> rowptr, fwd_rows, lptr, lpos, lcol, uptr, upos, dslot, pptr, pslot, ppos, err;  // factorisation
+  // sweeps: slots {row, first entry, end, -} grouped by level, entries {block
+  // position, column}
+  DevBuf<int4> fwd_slots, bwd_slots;
+  DevBuf<int2> lent, uent;
+  std::vector<int> fwd_off, bwd_off;
   DevBuf<signed char> kind;
   DevBuf<double> lu, dinv, tmp;
   // low-precision sweeps: float copies of the factors, made after each

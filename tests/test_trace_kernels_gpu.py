@@ -109,3 +109,42 @@ def test_gmres_against_a_dense_solve(n, restart):
         la.configure()
         la.solve()
         assert la.last_info[:2] == (its - 1, -3) and la.last_info[2] > 1e-11
+
+
+@pytest.mark.parametrize('ordering', [hf.linalg.PC_ILU0, hf.linalg.PC_ILU0_NATURAL], ids=['multicolour', 'natural'])
+@pytest.mark.parametrize('pattern', ['diagonal', 'one-way', 'lower', 'chain', 'dense'])
+def test_ilu_sweeps_on_odd_patterns(pattern, ordering):
+    """Patterns whose levels are degenerate: no off-diagonal entry at all (one level each way), entries without their
+    mirror image (a row that no row follows but a later row reads), a triangular matrix, a tridiagonal one and a dense
+    one.  No fill is dropped on any of them, so the preconditioner is the inverse and the solver stops within a few
+    steps (checked every 8) at the dense solution."""
+    print('ilu sweeps', pattern, ordering, flush=True)
+    rng = np.random.default_rng(3)
+    N = 41
+    A = np.diag(2.0 + rng.random(N))
+    if pattern == 'one-way':
+        A[1::3, 0] = 0.3
+        A[2::3, 1] = 0.2
+    elif pattern == 'lower':
+        A += 0.02 * np.tril(rng.random((N, N)), -1)
+    elif pattern == 'chain':
+        A += 0.4 * np.eye(N, k=1) + 0.3 * np.eye(N, k=-1)
+    elif pattern == 'dense':
+        A += 0.02 * rng.random((N, N))
+    b = rng.standard_normal(N)
+    la = hf.HipLinAlgebra(hf.HipOpts(solverType=hf.linalg.BCGS, preconditionnerType=ordering, rtol=1e-12, maxits=64))
+    la.initialize()
+    la.configure()
+    la.allocate(N)
+    for i in range(N):
+        cols = np.nonzero(A[i])[0]
+        la.setValsMatrix([i], cols, A[i, cols])
+    la.setValsRHS(np.arange(N), b)
+    la.assemble()
+    x = np.array(la.solve())
+    its, reason, rel = la.last_info
+    ref = np.linalg.solve(A, b)
+    assert reason == 2 and rel <= 1e-12
+    if pattern != 'chain' or ordering == hf.linalg.PC_ILU0_NATURAL:  # a recoloured chain drops fill
+        assert its <= 8
+    assert np.linalg.norm(x - ref) <= np.linalg.cond(A) * 1e-12 * np.linalg.norm(ref)
