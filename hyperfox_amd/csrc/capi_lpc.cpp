@@ -96,7 +96,7 @@ struct hfx_lpc {
     }
     if (nb == work_nb && E == work_E) return;
     acts.alloc(nb, E, L.O);
-    work.alloc(nb, E, L.O, 192LL * 64);
+    work.alloc(nb, E, L.O);
     zr.alloc((size_t)nb * L.bs);
     vr.alloc((size_t)nb * L.bs);
     lossacc.alloc(1);

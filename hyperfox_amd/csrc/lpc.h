@@ -79,9 +79,9 @@ struct LpcActs {
 
 // Gradient workspace.
 struct LpcGradWork {
-  DevBuf<float> dh, dh2, de, de2, dP, dX, dXn, dcn, dce, WT, part;
+  DevBuf<float> dh, dh2, de, de2, dP, dX, dXn, dcn, dce, part;
   int parts = 0;
-  void alloc(int nb, int E, int O, long long maxKN);
+  void alloc(int nb, int E, int O);
 };
 
 // FP32 forward pass; outputs in acts.cn / acts.ce (Dirichlet rows masked).

@@ -1,5 +1,5 @@
 // Kernels of the learned trace preconditioner (see lpc.h for the network and
-// the loss).  FP32 training path: LDS-tiled SIMT GEMMs with gathered inputs,
+// the loss).  FP32 training path: FP32 MFMA products with gathered inputs,
 // deterministic two-stage weight-gradient reductions, segmented row sums over
 // the BSR edge lists (no atomics anywhere, so a training run is bit
 // reproducible), Adam.  Inference: the same network on BF16 MFMA
@@ -93,7 +93,7 @@ namespace {
 
 constexpr int WG_PARTS = 256;
 
-void LpcGradWork_alloc(LpcGradWork& w, int nb, int E, int O, long long maxKN) {
+void LpcGradWork_alloc(LpcGradWork& w, int nb, int E, int O) {
   const size_t H = LPC_H, mx = (size_t)std::max(nb, E);
   w.dh.alloc((size_t)nb * H);
   w.dh2.alloc((size_t)nb * H);
@@ -104,7 +104,6 @@ void LpcGradWork_alloc(LpcGradWork& w, int nb, int E, int O, long long maxKN) {
   w.dXn.alloc((size_t)nb * 2 * H);
   w.dcn.alloc((size_t)nb * O);
   w.dce.alloc((size_t)std::max(E, 1) * O);
-  w.WT.alloc((size_t)maxKN);
   w.parts = WG_PARTS;
   w.part.alloc((size_t)WG_PARTS * (192 * 64 + 64));
 }
@@ -178,7 +177,8 @@ struct LinArgs {
   int rows = 0, nseg = 1;
   Seg seg[3];
   int K = 0;
-  const float* W = nullptr;  // W[k * ldw + n]
+  const float* W = nullptr;  // W[k * ldw + n], or (wt) W[n * ldw + k]
+  bool wt = false;
   int ldw = 0, ncols = 0;    // ncols <= 64
   const float* bias = nullptr;
   int act = 0;  // 1 = relu
@@ -208,77 +208,160 @@ __device__ __forceinline__ float gathered(const A& a, int r, int k) {
   return seg_at(a.seg[2], r, k);
 }
 
-// out[r, n] = act(sum_k X[r, k] W[k, n] + bias[n]), 64 x 64 output tiles,
-// 4 x 4 per thread, K in chunks of 32 through LDS.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// element q of lane group g <- element g of lane group q (groups of 16 lanes)
+__device__ __forceinline__ f32x4_t transpose4(f32x4_t x) {
+  typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+  unsigned u[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) u[q] = __float_as_uint(x[q]);
+  const u32x2_t a = __builtin_amdgcn_permlane32_swap(u[0], u[2], false, false);
+  const u32x2_t b = __builtin_amdgcn_permlane32_swap(u[1], u[3], false, false);
+  const u32x2_t c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const u32x2_t d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return f32x4_t{__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]), __uint_as_float(d[1])};
+}
+
+// out[r, n] = act(sum_k X[r, k] W[k, n] + bias[n]) on FP32 MFMA
+// (v_mfma_f32_16x16x4f32: FP32 products and sums).  A workgroup keeps its 64
+// columns of W in LDS, in the order of the MFMA operands, and takes 64-row
+// tiles: each wave 16 rows x 64 columns, four accumulators.  A lane reads four
+// consecutive inputs of one row per 16-deep chunk (rows are gathered through
+// index arrays, so nothing is staged), all NCH chunks at once, and the four
+// MFMA steps of a chunk multiply inputs 16 c + 4 q .. + 3 each, so the sum over
+// the inputs runs in their order, one fused multiply-add at a time (the
+// instruction's own order), as on one thread; a 4 x 4 transpose among the lane
+// groups turns the four consecutive inputs of a lane into the step's operands.
+// VEC: one segment of a multiple of 16, or segments of 64, 16-byte aligned;
+// otherwise the inputs are read one by one.  Bound by the gathered rows: 48,900 edges, 192 -> 64 (1.2 GFLOP, 63 MB):
+// 59 us with a 64 x 64 SIMT tile, 32 us.
+template <bool VEC, int NCH>
 __global__ __launch_bounds__(256) void lin_kernel(LinArgs a) {
-  __shared__ __align__(16) float Xs[32][68];
-  __shared__ __align__(16) float Ws[32][64];
-  const int t = threadIdx.x, tn = t & 15, tm = t >> 4;
+  extern __shared__ __align__(16) float Wl[];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 15, lg = lane >> 4;
+  const int c0 = blockIdx.y * 64, ncols = min(64, a.ncols - c0);
   const int ntiles = (a.rows + 63) >> 6;
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int r0 = tile << 6;
-    float acc[4][4];
+  f32x4_t x[NCH];
+  auto inputs = [&](int tile) {
+    const int rr = min((tile << 6) + wave * 16 + li, a.rows - 1);  // rows past the end repeat the last one
+    const float* ps[3];  // 64 inputs each (one wide segment is cut into pieces of 64)
+    if constexpr (VEC) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-    for (int k0 = 0; k0 < a.K; k0 += 32) {
-      for (int e = t; e < 2048; e += 256) {
-        const int row = e >> 5, kk = e & 31, r = r0 + row, k = k0 + kk;
-        Xs[kk][row] = (r < a.rows && k < a.K) ? gathered(a, r, k) : 0.f;
+      for (int g = 0; g < (NCH + 3) / 4; ++g) {
+        const Seg& sg = a.seg[g < a.nseg ? g : 0];
+        ps[g] = sg.p + (long long)(sg.idx ? sg.idx[rr] : rr) * sg.ld + (a.nseg == 1 ? g * 64 : 0);
       }
-      for (int e = t; e < 2048; e += 256) {
-        const int kk = e >> 6, n = e & 63, k = k0 + kk;
-        Ws[kk][n] = (k < a.K && n < a.ncols) ? a.W[(long long)k * a.ldw + n] : 0.f;
-      }
-      __syncthreads();
-#pragma unroll 8
-      for (int kk = 0; kk < 32; ++kk) {
-        const float4 xv = *reinterpret_cast<const float4*>(&Xs[kk][tm * 4]);
-        const float4 wv = *reinterpret_cast<const float4*>(&Ws[kk][tn * 4]);
-        const float xs[4] = {xv.x, xv.y, xv.z, xv.w}, ws[4] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] += xs[i] * ws[j];
-      }
-      __syncthreads();
     }
 #pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      if constexpr (VEC) {
+        x[c] = c * 16 < a.K ? *reinterpret_cast<const f32x4_t*>(ps[c / 4] + (c % 4) * 16 + lg * 4)
+                            : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int kq = c * 16 + q * 4 + lg;
+          x[c][q] = kq < a.K ? gathered(a, rr, kq) : 0.f;
+        }
+      }
+    }
+  };
+  if ((int)blockIdx.x < ntiles) inputs(blockIdx.x);  // on their way while W is staged
+  {
+    // W four columns at a time (transposed: four rows), 16 loads in flight
+    constexpr int SG = NCH < 4 ? NCH : 4;
+    for (int e0 = 0; e0 < NCH; e0 += SG) {
+      float wv[SG][4];
+#pragma unroll
+      for (int e = 0; e < SG; ++e)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int k = (e0 + e) * 16 + (a.wt ? (t & 3) * 4 + j : t >> 4), n = a.wt ? t >> 2 : (t & 15) * 4 + j;
+          const bool on = k < a.K && n < ncols;
+          const int kc = on ? k : 0, nc = c0 + (on ? n : 0);
+          const float v = a.W[a.wt ? nc * a.ldw + kc : kc * a.ldw + nc];
+          wv[e][j] = on ? v : 0.f;
+        }
+#pragma unroll
+      for (int e = 0; e < SG; ++e)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int k = a.wt ? (t & 3) * 4 + j : t >> 4, n = a.wt ? t >> 2 : (t & 15) * 4 + j;
+          Wl[(((e0 + e) * 4 + (k & 3)) * 64 + n) * 4 + ((k >> 2) & 3)] = wv[e][j];
+        }
+    }
+  }
+  __syncthreads();
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int r0 = (tile << 6) + wave * 16;
+    asm volatile("" ::: "memory");  // W is read again for every tile, not kept in registers (and spilled) across them
+    f32x4_t acc[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      if constexpr (VEC) x[c] = transpose4(x[c]);
+      f32x4_t w[4];
+#pragma unroll
+      for (int n = 0; n < 4; ++n) w[n] = *reinterpret_cast<const f32x4_t*>(Wl + ((c * 4 + lg) * 64 + n * 16 + li) * 4);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[c][q], w[n][q], acc[n], 0, 0, 0);
+    }
+    // result row 4 (lane / 16) + i, column lane % 16 in accumulator element i
+#pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = r0 + tm * 4 + i;
+      const int r = r0 + lg * 4 + i;
       if (r >= a.rows) continue;
       const bool masked = a.rowmask && a.rowmask[a.maskidx ? a.maskidx[r] : r];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = tn * 4 + j;
-        if (n >= a.ncols) continue;
-        float v = acc[i][j] + (a.bias ? a.bias[n] : 0.f);
+      for (int nt = 0; nt < 4; ++nt) {
+        const int n = nt * 16 + li;
+        if (n >= ncols) continue;
+        float v = acc[nt][i] + (a.bias ? a.bias[c0 + n] : 0.f);
         if (a.act) v = fmaxf(v, 0.f);
         if (masked) v = 0.f;
-        a.out[(long long)r * a.ldo + n] = v;
-        if (a.out2) a.out2[(long long)r * a.ldo2 + n] = a.res[(long long)r * a.ldr + n] + v;
+        a.out[(long long)r * a.ldo + c0 + n] = v;
+        if (a.out2) a.out2[(long long)r * a.ldo2 + c0 + n] = a.res[(long long)r * a.ldr + c0 + n] + v;
       }
     }
+    if (tile + (int)gridDim.x < ntiles) inputs(tile + gridDim.x);
   }
 }
 
-// Launch lin_kernel over all output columns in chunks of 64.
+// Inputs that the kernels may read in 16-byte pieces of 64 per segment: one
+// segment of a multiple of 16, or segments of 64
+bool segs_vec(int nseg, const Seg* seg) {
+  for (int g = 0; g < nseg; ++g)
+    if (seg[g].w % 16 != 0 || (nseg > 1 && seg[g].w != 64) || seg[g].ld % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(seg[g].p) % 16 != 0)
+      return false;
+  return true;
+}
+
+// Launch lin_kernel over all N output columns, 64 to a workgroup.
 void lin(LinArgs a, int N, hipStream_t s) {
   if (a.rows <= 0) return;
-  const int ntiles = (a.rows + 63) / 64;
-  const int grid = std::min(ntiles, 4096);
-  for (int c0 = 0; c0 < N; c0 += 64) {
-    LinArgs b = a;
-    b.ncols = std::min(64, N - c0);
-    b.W = a.W + c0;
-    if (a.bias) b.bias = a.bias + c0;
-    b.out = a.out + c0;
-    if (a.res) b.res = a.res + c0;
-    if (a.out2) b.out2 = a.out2 + c0;
-    hipLaunchKernelGGL(lin_kernel, dim3(grid), dim3(256), 0, s, b);
-    HFX_HIP(hipGetLastError());
-  }
+  if (a.K > 192) throw std::runtime_error("learned preconditioner: layer input wider than 192");
+  a.ncols = N;
+  const int ntiles = (a.rows + 63) / 64, nch = (a.K + 15) / 16;
+  const dim3 grid(std::min(ntiles, 2048), (N + 63) / 64);
+  const bool vec = segs_vec(a.nseg, a.seg);
+  auto go = [&](auto kern, int chunks) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), (size_t)chunks * 1024 * sizeof(float), s, a);
+  };
+#define HFX_NCH(C) \
+  if (vec) go(lin_kernel<true, C>, C); \
+  else go(lin_kernel<false, C>, C);
+  if (nch <= 1) { HFX_NCH(1) }
+  else if (nch <= 2) { HFX_NCH(2) }
+  else if (nch <= 4) { HFX_NCH(4) }
+  else if (nch <= 8) { HFX_NCH(8) }
+  else { HFX_NCH(12) }
+#undef HFX_NCH
+  HFX_HIP(hipGetLastError());
 }
 
 // ------------------------------------------------------ weight gradients
@@ -293,54 +376,153 @@ struct WgArgs {
   int rows_per_part = 0;
 };
 
-// Partial dW = X^T dP and db = sum dP over this block's rows; thread (n, g)
-// owns column n and rows k = g, g+4, ... of dW.
+// Partial dW = X^T dP and db = sum dP over this block's rows, on FP32 MFMA with
+// the rows as the summed index: lane (i, g) supplies X[r + g][16 kt + i] and
+// dP[r + g][16 nt + i], so operands come straight from memory, and one wave
+// holds the whole KT x 4 tiles of dW.  The waves take every fourth group of
+// four rows (the next group's operands are read while the current one is
+// multiplied) and add up in LDS, wave by wave.  KT: tiles of 16 inputs.
+// 48,900 edges, 192 x 64: 126 us with one column per thread (an LDS read per
+// multiply-add), 37 us.
+template <bool VEC, int KT>
 __global__ __launch_bounds__(256) void wgrad_kernel(WgArgs a) {
-  __shared__ float Xs[32][193];
-  __shared__ float Ps[32][64];
-  const int t = threadIdx.x, n = t & 63, g = t >> 6;
-  float acc[48];
-#pragma unroll
-  for (int j = 0; j < 48; ++j) acc[j] = 0.f;
-  float accb = 0.f;
+  __shared__ float sw[KT * 16 * 64 + 64];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 15, lg = lane >> 4;
   const int rbeg = blockIdx.x * a.rows_per_part;
   const int rend = min(a.rows, rbeg + a.rows_per_part);
-  for (int c0 = rbeg; c0 < rend; c0 += 32) {
-    for (int e = t; e < 32 * 192; e += 256) {
-      const int row = e / 192, k = e - row * 192, r = c0 + row;
-      Xs[row][k] = (r < rend && k < a.K) ? gathered(a, r, k) : 0.f;
-    }
-    for (int e = t; e < 32 * 64; e += 256) {
-      const int row = e >> 6, nn = e & 63, r = c0 + row;
-      Ps[row][nn] = (r < rend && nn < a.ncols) ? a.dP[(long long)r * a.ldp + nn] : 0.f;
-    }
-    __syncthreads();
-    for (int row = 0; row < 32; ++row) {
-      const float d = Ps[row][n];
-      accb += d;
+  f32x4_t acc[KT][4];
+  float accb[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 48; ++j) acc[j] += Xs[row][g + 4 * j] * d;
+  for (int k = 0; k < KT; ++k)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[k][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // RG groups of four rows per step; the rows' indices are read a step before
+  // their inputs, those a step before their products
+  constexpr int RG = 2;
+  struct Rows {
+    int i[3][RG];
+  };
+  auto indices = [&](int r0, Rows& ix) {
+#pragma unroll
+    for (int u = 0; u < RG; ++u) {
+      const int r = r0 + u * 16 + lg, rc = r < rend ? r : rbeg;
+#pragma unroll
+      for (int g = 0; g < 3; ++g) ix.i[g][u] = g < a.nseg && a.seg[g].idx ? a.seg[g].idx[rc] : rc;
+    }
+  };
+  auto operands = [&](int r0, const Rows& ix, float (*x)[KT], float (*d)[4]) {
+#pragma unroll
+    for (int u = 0; u < RG; ++u) {
+      const int r = r0 + u * 16 + lg;
+      const bool on = r < rend;
+      const int rc = on ? r : rbeg;
+      if constexpr (VEC) {
+        const float* p[3];
+#pragma unroll
+        for (int g = 0; g < (KT + 3) / 4; ++g) {
+          const Seg& sg = a.seg[g < a.nseg ? g : 0];
+          p[g] = sg.p + (long long)ix.i[g < a.nseg ? g : 0][u] * sg.ld + (a.nseg == 1 ? g * 64 : 0) + li;
+        }
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          const float v = kt * 16 < a.K ? p[kt / 4][(kt % 4) * 16] : 0.f;
+          x[u][kt] = on ? v : 0.f;
+        }
+      } else {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          const int k = kt * 16 + li;
+          x[u][kt] = on && k < a.K ? gathered(a, rc, k) : 0.f;
+        }
+      }
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) {
+        const int n = nt * 16 + li;
+        const float v = a.dP[(long long)rc * a.ldp + (n < a.ncols ? n : 0)];
+        d[u][nt] = on && n < a.ncols ? v : 0.f;
+      }
+    }
+  };
+  float x[RG][KT], d[RG][4], xn[RG][KT], dn[RG][4];
+  Rows ix;
+  constexpr int STEP = 16 * RG;
+  int r0 = rbeg + wave * 4;
+  indices(r0, ix);
+  if (r0 < rend) operands(r0, ix, x, d);
+  indices(r0 + STEP, ix);
+  for (; r0 < rend; r0 += STEP) {
+    if (r0 + STEP < rend) operands(r0 + STEP, ix, xn, dn);
+    indices(r0 + 2 * STEP, ix);
+#pragma unroll
+    for (int u = 0; u < RG; ++u)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+          acc[kt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u][kt], d[u][nt], acc[kt][nt], 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < RG; ++u) {
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) {
+        accb[nt] += d[u][nt];
+        d[u][nt] = dn[u][nt];
+      }
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) x[u][kt] = xn[u][kt];
+    }
+  }
+  // db: the four row groups of a lane column
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) {
+    accb[nt] += __shfl_xor(accb[nt], 16, 64);
+    accb[nt] += __shfl_xor(accb[nt], 32, 64);
+  }
+  // tile (kt, nt), element i of lane l at ((kt 4 + nt) 4 + i) 64 + l
+  for (int w = 0; w < 4; ++w) {
+    if (wave == w) {
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float* o = sw + ((kt * 4 + nt) * 4 + i) * 64 + lane;
+            *o = w == 0 ? acc[kt][nt][i] : *o + acc[kt][nt][i];
+          }
+      if (lg == 0)
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+          float* o = sw + KT * 16 * 64 + nt * 16 + li;
+          *o = w == 0 ? accb[nt] : *o + accb[nt];
+        }
     }
     __syncthreads();
   }
-  if (n >= a.ncols) return;
   float* p = a.part + (size_t)blockIdx.x * (a.K * a.ncols + a.ncols);
-#pragma unroll
-  for (int j = 0; j < 48; ++j) {
-    const int k = g + 4 * j;
-    if (k < a.K) p[k * a.ncols + n] = acc[j];
+  for (int e = t; e < a.K * a.ncols; e += 256) {
+    const int k = e / a.ncols, n = e % a.ncols;  // result row 4 (lane / 16) + i, column lane % 16
+    p[e] = sw[(((k >> 4) * 4 + (n >> 4)) * 4 + (k & 3)) * 64 + ((k >> 2) & 3) * 16 + (n & 15)];
   }
-  if (g == 0) p[a.K * a.ncols + n] = accb;
+  for (int e = t; e < a.ncols; e += 256) p[a.K * a.ncols + e] = sw[KT * 16 * 64 + e];
 }
 
-__global__ void wgrad_reduce_kernel(int parts, int K, int ncols, const float* __restrict__ part, float* __restrict__ gW,
-                                    int ldw, float* __restrict__ gb) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+// Sum of the parts: 64 outputs to a workgroup, its four waves take every
+// fourth part (with one output per thread and all parts in a row this was 53 us
+// of a 75 us gradient).
+__global__ __launch_bounds__(256) void wgrad_reduce_kernel(int parts, int K, int ncols, const float* __restrict__ part,
+                                                           float* __restrict__ gW, int ldw, float* __restrict__ gb) {
+  __shared__ float red[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = blockIdx.x * 64 + lane;
   const int tot = K * ncols + ncols;
-  if (t >= tot) return;
-  const size_t stride = (size_t)tot;
   float acc = 0.f;
-  for (int b = 0; b < parts; ++b) acc += part[b * stride + t];
+  if (t < tot) {
+#pragma unroll 8
+    for (int b = wave; b < parts; b += 4) acc += part[(size_t)b * tot + t];
+  }
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave != 0 || t >= tot) return;
+  acc = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
   if (t < K * ncols) gW[(t / ncols) * ldw + (t % ncols)] = acc;
   else gb[t - K * ncols] = acc;
 }
@@ -365,10 +547,21 @@ void wgrad(WgArgs a, int N, float* gW, float* gb, float* part, hipStream_t s) {
     b.dP = a.dP + c0;
     b.part = part;
     b.rows_per_part = rpp;
-    hipLaunchKernelGGL(wgrad_kernel, dim3(used), dim3(256), 0, s, b);
+    const int kt = (b.K + 15) / 16;
+    const bool vec = segs_vec(b.nseg, b.seg);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(used), dim3(256), 0, s, b); };
+#define HFX_KT(T) \
+    if (vec) go(wgrad_kernel<true, T>); \
+    else go(wgrad_kernel<false, T>);
+    if (kt <= 1) { HFX_KT(1) }
+    else if (kt <= 2) { HFX_KT(2) }
+    else if (kt <= 4) { HFX_KT(4) }
+    else if (kt <= 8) { HFX_KT(8) }
+    else { HFX_KT(12) }
+#undef HFX_KT
     HFX_HIP(hipGetLastError());
     const int tot = b.K * b.ncols + b.ncols;
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(ceil_div(tot, 256)), dim3(256), 0, s, used, b.K, b.ncols, part,
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(ceil_div(tot, 64)), dim3(256), 0, s, used, b.K, b.ncols, part,
                        gW + c0, N, gb + c0);
     HFX_HIP(hipGetLastError());
   }
@@ -423,18 +616,6 @@ __global__ void add_strided_kernel(int rows, const float* __restrict__ a, const 
   if (t >= (long long)rows * LPC_H) return;
   const int r = (int)(t / LPC_H), c = (int)(t % LPC_H);
   out[t] = a[t] + b[(long long)r * ldb + off + c];
-}
-
-__global__ void transpose_kernel(int K, int N, const float* __restrict__ W, float* __restrict__ WT) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= K * N) return;
-  const int k = t / N, n = t % N;
-  WT[n * K + k] = W[t];
-}
-
-void transpose(int K, int N, const float* W, float* WT, hipStream_t s) {
-  hipLaunchKernelGGL(transpose_kernel, dim3(ceil_div(K * N, 256)), dim3(256), 0, s, K, N, W, WT);
-  HFX_HIP(hipGetLastError());
 }
 
 __global__ void fill_kernel(long long n, float v, float* __restrict__ p) {
@@ -793,7 +974,7 @@ void forward_impl(const LpcLayout& L, const float* P, const unsigned short* W16,
 
 }  // namespace
 
-void LpcGradWork::alloc(int nb, int E, int O, long long maxKN) { LpcGradWork_alloc(*this, nb, E, O, maxKN); }
+void LpcGradWork::alloc(int nb, int E, int O) { LpcGradWork_alloc(*this, nb, E, O); }
 
 void LpcSystem::build(const LpcGraph& g, const double* vals, hipStream_t s) {
   const int bs = g.bs;
@@ -921,24 +1102,24 @@ void lpc_backward(const LpcLayout& L, const float* P, const LpcGraph& g, const L
   float* de = w.de.p;
   float* de2 = w.de2.p;
   {
-    transpose(H, O, P + L.Wdn, w.WT.p, s);
     LinArgs a;
     a.rows = nb;
     a.seg[0] = seg(w.dcn.p, nullptr, O, O);
     a.K = O;
-    a.W = w.WT.p;
-    a.ldw = H;
+    a.W = P + L.Wdn;
+    a.wt = true;
+    a.ldw = O;
     a.out = dh;
     a.ldo = H;
     lin(a, H, s);
     if (E > 0) {
-      transpose(H, O, P + L.Wde, w.WT.p, s);
       LinArgs b;
       b.rows = E;
       b.seg[0] = seg(w.dce.p, nullptr, O, O);
       b.K = O;
-      b.W = w.WT.p;
-      b.ldw = H;
+      b.W = P + L.Wde;
+      b.wt = true;
+      b.ldw = O;
       b.out = de;
       b.ldo = H;
       lin(b, H, s);
@@ -960,14 +1141,14 @@ void lpc_backward(const LpcLayout& L, const float* P, const LpcGraph& g, const L
       a.ldp = H;
       wgrad(a, H, grad + L.Wu[l], grad + L.bu[l], part, s);
     }
-    transpose(2 * H, H, P + L.Wu[l], w.WT.p, s);
     {
       LinArgs a;
       a.rows = nb;
       a.seg[0] = seg(w.dP.p, nullptr, H, H);
       a.K = H;
-      a.W = w.WT.p;
-      a.ldw = 2 * H;
+      a.W = P + L.Wu[l];
+      a.wt = true;
+      a.ldw = H;
       a.out = w.dXn.p;
       a.ldo = 2 * H;
       lin(a, 2 * H, s);
@@ -992,14 +1173,14 @@ void lpc_backward(const LpcLayout& L, const float* P, const LpcGraph& g, const L
         a.ldp = H;
         wgrad(a, H, grad + L.Wm[l], grad + L.bm[l], part, s);
       }
-      transpose(3 * H, H, P + L.Wm[l], w.WT.p, s);
       {
         LinArgs a;
         a.rows = E;
         a.seg[0] = seg(w.dP.p, nullptr, H, H);
         a.K = H;
-        a.W = w.WT.p;
-        a.ldw = 3 * H;
+        a.W = P + L.Wm[l];
+        a.wt = true;
+        a.ldw = H;
         a.out = w.dX.p;
         a.ldo = 3 * H;
         lin(a, 3 * H, s);
