@@ -61,7 +61,8 @@ using hfx::pack_tables;
 
 // Reference tables of the affine element kernel (order of ALay in
 // hdg_affine.hip): PHI, DPHI, FPHI, W, FW, Ahat_a = Mhat^-1 Chat_a,
-// G_g = Mhat^-1[:, fn_g] Mfhat.  Built in long double.
+// G_g = Mhat^-1[:, fn_g] Mfhat, and Mhat^-1 (read by the explicit stage kernel
+// only).  Built in long double.
 void pack_affine_tables(const hfx::RefEl& re, std::vector<double>& t) {
   const int d = re.dim, nN = re.nN, nip = re.nip();
   const hfx::RefEl& fe = *re.face;
@@ -111,6 +112,7 @@ void pack_affine_tables(const hfx::RefEl& re, std::vector<double>& t) {
         for (int a2 = 0; a2 < nNf; ++a2) s += Mi[j * nN + re.faceNodes[g][a2]] * Mf[a2 * nNf + b];
         t.push_back((double)s);
       }
+  for (const ld v : Mi) t.push_back((double)v);
 }
 
 // True when every cell's nodes are the affine image of its vertices (so

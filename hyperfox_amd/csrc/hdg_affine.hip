@@ -1269,6 +1269,10 @@ constexpr int aff_wave_fit() {
 
 void launch_affine(int dim, int order, bool tensor_d, int waves, const ElemArgs& a, int grid_cap, hipStream_t s) {
   if (tensor_d) throw std::runtime_error("affine element kernel: tensor diffusion uses the general kernel");
+  if (explicit_stage(a)) {
+    launch_explicit_stage(dim, order, a, grid_cap, s);
+    return;
+  }
   if (a.ts_gen) {
     // the time-transform variant exists at the LDS-fitting wave count only
 #define HFX_CASE(D, P)                                                                     \

@@ -115,6 +115,12 @@ size_t element_workspace_doubles(int dim, int order);
 void launch_affine(int dim, int order, bool tensor_d, int waves, const ElemArgs& a, int grid_cap, hipStream_t s);
 size_t affine_lds_bytes(int dim, int order, bool tensor_d, int waves);
 
+// A Runge-Kutta stage whose model rows drop out (a_ss = 0) in an explicit HDG
+// mode needs no condensation: launch_affine hands such arguments to the kernel
+// of hdg_explicit.hip (same tables, outputs and scatter).
+bool explicit_stage(const ElemArgs& a);
+void launch_explicit_stage(int dim, int order, const ElemArgs& a, int grid_cap, hipStream_t s);
+
 // One work item of the batched affine kernels: cells [e0, e1) of problem
 // `prob` (index into the ElemArgs table) of order `order` (2-D).
 struct BatchItem {
