@@ -91,22 +91,75 @@ constexpr bool element_in_workspace() {
   return (size_t)Layout<D, P, 64>::TOTAL * sizeof(double) > 160 * 1024;
 }
 
+// The two eliminations touch every entry of their matrices once a step, so
+// the workspace orders hold those in LDS: both, where both fit (2-D p 7 to 9,
+// 3-D p = 4), else the one at work, copied in and out (2-D p = 10, 3-D p = 5).
+// The tables are read where they are (one copy for every workgroup) and the
+// IP data lies in LDS too: a slab of 286 KB per workgroup, 18 MB for the 64
+// workgroups of an XCD, went through its 4 MB of L2 for every phase.
+// Measured, 1,296 3-D p=4 cells: 4.48 ms with everything in the workspace,
+// 2.81 ms with the matrices in LDS and two workgroups per CU, 1.93 ms with the
+// rest.
+template <int D, int P>
+struct ElemLds {
+  using L = Layout<D, P, 64>;
+  static constexpr int A1 = L::NN * L::NC1, A2 = L::NN * L::NC2;
+  static constexpr bool WS = element_in_workspace<D, P>();
+  static constexpr bool BOTH = (size_t)(A1 + A2) * sizeof(double) <= 156 * 1024;
+  // Phase 1 (gathered inputs and IP data, without the gradients, which are
+  // formed from the tables where they are used) is over before AUG2 is filled
+  // (BOTH) or AUG1 copied in, and lies in their place.
+  static constexpr int O_P1 = BOTH ? A1 : 0;
+  static constexpr int N_P1 = (L::O_GR - L::O_X) + L::NF * L::NIPF * L::NS;
+  static_assert(!WS || N_P1 <= (BOTH ? A2 : A1), "phase 1 does not fit its overlay");
+  static constexpr size_t BYTES = (size_t)(!WS ? L::TOTAL : BOTH ? A1 + A2 : A1 > A2 ? A1 : A2) * sizeof(double);
+};
+
+// Waves per SIMD that the registers are held to.  Left alone the kernel takes
+// up to 350, one wave per SIMD, and a workgroup of four leaves no second one
+// beside it (7,442 2-D p=3 cells with a tensor: 0.376 ms so, 0.264 ms with two).
+constexpr int ELEMENT_WAVES = 2;
+
+// Columns of the volume blocks per thread: as few as let one pass of the
+// workgroup cover them, at most 5 (their sums stay in registers).
+constexpr int volume_columns(int nn, int nt) {
+  int jb = 1;
+  while (jb < 5 && nn * ((nn + jb - 1) / jb) > nt) ++jb;
+  return jb;
+}
+
+// gauss_jordan on a workspace matrix through the LDS buffer
+template <int NR, int NC, int NT>
+__device__ void gauss_jordan_via(double* A, double* lds, int* perm) {
+  for (int t = threadIdx.x; t < NR * NC; t += NT) lds[t] = A[t];
+  __syncthreads();
+  gauss_jordan<NR, NC, NT>(lds, perm);
+  for (int t = threadIdx.x; t < NR * (NC - NR); t += NT) {
+    const int o = (t / (NC - NR)) * NC + NR + t % (NC - NR);
+    A[o] = lds[o];
+  }
+  __syncthreads();
+}
+
 template <int D, int P, int NT>
-__global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(ELEMENT_WAVES)))
+void hdg_element_kernel(ElemArgs a) {
   using L = Layout<D, P, NT>;
   using Z = ESz<D, P>;
   constexpr int NN = L::NN, NNF = L::NNF, NIP = L::NIP, NIPF = L::NIPF, NF = L::NF, NL = L::NL, NS = L::NS;
   constexpr int NC1 = L::NC1, NC2 = L::NC2;
   extern __shared__ double lds_ws[];
   double* sm = lds_ws;
-  if constexpr (element_in_workspace<D, P>()) sm = a.gws + (size_t)blockIdx.x * L::TOTAL;
+  using E = ElemLds<D, P>;
+  if constexpr (E::WS) sm = a.gws + (size_t)blockIdx.x * L::TOTAL;
   __shared__ int fn[NF * NNF];
   __shared__ int pos[NF * NN];
   __shared__ int vopp[NF];
   __shared__ int perm1[NN], perm2[NN];
   const int tid = threadIdx.x;
 
-  for (int t = tid; t < Z::TAB; t += NT) sm[L::O_TAB + t] = a.tabs[t];
+  if constexpr (!E::WS)
+    for (int t = tid; t < Z::TAB; t += NT) sm[L::O_TAB + t] = a.tabs[t];
   for (int t = tid; t < NF * NN; t += NT) pos[t] = -1;
   __syncthreads();
   for (int t = tid; t < NF * NNF; t += NT) {
@@ -122,30 +175,32 @@ __global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
   }
   __syncthreads();
 
-  const double* PHI = sm + L::O_TAB + Z::T_PHI;
-  const double* DPHI = sm + L::O_TAB + Z::T_DPHI;
-  const double* FPHI = sm + L::O_TAB + Z::T_FPHI;
-  const double* FDPHI = sm + L::O_TAB + Z::T_FDPHI;
-  const double* W = sm + L::O_TAB + Z::T_W;
-  const double* FW = sm + L::O_TAB + Z::T_FW;
+  const double* TB = E::WS ? a.tabs : sm + L::O_TAB;
+  const double* PHI = TB + Z::T_PHI;
+  const double* DPHI = TB + Z::T_DPHI;
+  const double* FPHI = TB + Z::T_FPHI;
+  const double* FDPHI = TB + Z::T_FDPHI;
+  const double* W = TB + Z::T_W;
+  const double* FW = TB + Z::T_FW;
   double* FM = sm + L::O_FM;
-  double* AUG1 = sm + L::O_AUG1;
-  double* AUG2 = sm + L::O_AUG2;
+  double* AUG1 = E::WS && E::BOTH ? lds_ws : sm + L::O_AUG1;
+  double* AUG2 = E::WS && E::BOTH ? lds_ws + E::A1 : sm + L::O_AUG2;
   double* SUQ = sm + L::O_SUQ;
   double* SUU = sm + L::O_SUU;
   double* FU = sm + L::O_FU;
-  double* X = sm + L::O_X;
-  double* DN = sm + L::O_DN;
-  double* BN = sm + L::O_BN;
-  double* TAU = sm + L::O_TAU;
-  double* FQ = sm + L::O_FQ;
-  double* RQ = sm + L::O_RQ;
-  double* DV = sm + L::O_DV;
-  double* JI = sm + L::O_JI;
-  double* DQ = sm + L::O_DQ;
-  double* BQ = sm + L::O_BQ;
-  double* GR = sm + L::O_GR;
-  double* FWT = sm + L::O_FWT;
+  double* P1 = E::WS ? lds_ws + E::O_P1 : sm + L::O_X;
+  double* X = P1;
+  double* DN = P1 + (L::O_DN - L::O_X);
+  double* BN = P1 + (L::O_BN - L::O_X);
+  double* TAU = P1 + (L::O_TAU - L::O_X);
+  double* FQ = P1 + (L::O_FQ - L::O_X);
+  double* RQ = P1 + (L::O_RQ - L::O_X);
+  double* DV = P1 + (L::O_DV - L::O_X);
+  double* JI = P1 + (L::O_JI - L::O_X);
+  double* DQ = P1 + (L::O_DQ - L::O_X);
+  double* BQ = P1 + (L::O_BQ - L::O_X);
+  double* GR = sm + L::O_GR;  // not in the workspace orders
+  double* FWT = P1 + ((E::WS ? L::O_GR : L::O_FWT) - L::O_X);
   double* ZB = sm + L::O_Z;
   double* QL = sm + L::O_QL;
   double* Q0L = sm + L::O_Q0L;
@@ -185,26 +240,24 @@ __global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
       RQ[t] = (a.hasR ? a.r_ip[(size_t)e * NIP + t] : 0.0) + a.ts_idt;
     }
     __syncthreads();
-    // ---------------------------------------------- IP geometry (element)
-    for (int q = tid; q < NIP; q += NT) {
-      double J[D * D];
-      for (int t = 0; t < D * D; ++t) J[t] = 0.0;
-      for (int i = 0; i < NN; ++i)
-        for (int r = 0; r < D; ++r)
-          for (int c = 0; c < D; ++c) J[r * D + c] += DPHI[(q * NN + i) * D + r] * X[i * D + c];
-      double dt = det_small<D>(J);
-      DV[q] = W[q] * dt;
-      inv_small<D>(J, dt, JI + q * D * D);
-      for (int t = 0; t < D * D; ++t) {
-        double s = 0.0;
-        for (int i = 0; i < NN; ++i) s += PHI[q * NN + i] * DN[i * D * D + t];
-        DQ[q * D * D + t] = s;
+    // ------------------------- IP fields: J (into JI), D, b, one entry each
+    constexpr int NG = 2 * D * D + D;
+    for (int t = tid; t < NIP * NG; t += NT) {
+      const int q = t / NG, c = t % NG;
+      const double *row, *src;
+      double* dst;
+      int rs, ss;
+      if (c < D * D) {
+        row = DPHI + q * NN * D + c / D; rs = D; src = X + c % D; ss = D; dst = JI + q * D * D + c;
+      } else if (c < 2 * D * D) {
+        row = PHI + q * NN; rs = 1; src = DN + (c - D * D); ss = D * D; dst = DQ + q * D * D + (c - D * D);
+      } else {
+        row = PHI + q * NN; rs = 1; src = BN + (c - 2 * D * D); ss = D; dst = BQ + q * D + (c - 2 * D * D);
       }
-      for (int k = 0; k < D; ++k) {
-        double s = 0.0;
-        for (int i = 0; i < NN; ++i) s += PHI[q * NN + i] * BN[i * D + k];
-        BQ[q * D + k] = s;
-      }
+      double s = 0.0;
+#pragma unroll 4
+      for (int i = 0; i < NN; ++i) s += row[i * rs] * src[i * ss];
+      *dst = s;
     }
     // ------------------------------------------------- IP geometry (faces)
     for (int t = tid; t < NF * NIPF; t += NT) {
@@ -269,8 +322,16 @@ __global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
       }
     }
     __syncthreads();
+    for (int q = tid; q < NIP; q += NT) {
+      double J[D * D];
+      for (int t = 0; t < D * D; ++t) J[t] = JI[q * D * D + t];
+      const double dt = det_small<D>(J);
+      DV[q] = W[q] * dt;
+      inv_small<D>(J, dt, JI + q * D * D);
+    }
+    __syncthreads();
     // physical gradients GR[q][i][k] = (J^-1 grad_xi phi_i)_k
-    for (int t = tid; t < NIP * NN; t += NT) {
+    for (int t = tid; t < (E::WS ? 0 : NIP * NN); t += NT) {
       int q = t / NN, i = t % NN;
       for (int k = 0; k < D; ++k) {
         double s = 0.0;
@@ -278,52 +339,85 @@ __global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
         GR[t * D + k] = s;
       }
     }
-    // weighted face masses
-    for (int t = tid; t < NF * NS * NNF * NNF; t += NT) {
-      int b = t % NNF, aa = (t / NNF) % NNF, s = (t / (NNF * NNF)) % NS, f = t / (NS * NNF * NNF);
-      double acc = 0.0;
-      for (int q = 0; q < NIPF; ++q) acc += FWT[(f * NIPF + q) * NS + s] * FPHI[q * NNF + aa] * FPHI[q * NNF + b];
-      FM[t] = acc;
+    // weighted face masses, every weight of one (f, a, b) by one thread
+    for (int t = tid; t < NF * NNF * NNF; t += NT) {
+      const int b = t % NNF, aa = (t / NNF) % NNF, f = t / (NNF * NNF);
+      double acc[NS];
+      for (int s = 0; s < NS; ++s) acc[s] = 0.0;
+#pragma unroll 2
+      for (int q = 0; q < NIPF; ++q) {
+        const double pa = FPHI[q * NNF + aa], pb = FPHI[q * NNF + b];
+        const double* w = FWT + (f * NIPF + q) * NS;
+        for (int s = 0; s < NS; ++s) acc[s] += w[s] * pa * pb;
+      }
+      for (int s = 0; s < NS; ++s) FM[((f * NS + s) * NNF + aa) * NNF + b] = acc[s];
     }
     __syncthreads();
     // -------------------------------------------------- volume blocks
-    for (int t = tid; t < NN * NN; t += NT) {
-      const int i = t / NN, j = t % NN;
-      double m = 0.0, suu = 0.0, cg[D], sq[D];
-      for (int k = 0; k < D; ++k) { cg[k] = 0.0; sq[k] = 0.0; }
+    constexpr int JB = volume_columns(NN, NT), JG = (NN + JB - 1) / JB;  // JB columns per thread share row i's part
+    for (int t = tid; t < NN * JG; t += NT) {
+      const int i = t / JG, j0 = t % JG;
+      double m[JB], suu[JB], cg[JB][D], sq[JB][D];
+      int ju[JB];
+#pragma unroll
+      for (int u = 0; u < JB; ++u) {
+        ju[u] = j0 + u * JG < NN ? j0 + u * JG : NN - 1;
+        m[u] = suu[u] = 0.0;
+        for (int k = 0; k < D; ++k) cg[u][k] = sq[u][k] = 0.0;
+      }
+#pragma unroll 1
       for (int q = 0; q < NIP; ++q) {
-        const double w = DV[q];
-        const double pi = PHI[q * NN + i], pj = w * PHI[q * NN + j];
-        const double* g = GR + (q * NN + i) * D;
-        m += pi * pj;
-        double bg = 0.0;
+        const double w = DV[q], pi = PHI[q * NN + i];
+        double g[D], dg[D], bg = 0.0;
         for (int k = 0; k < D; ++k) {
-          cg[k] += g[k] * pj;
-          double s = 0.0;
-          for (int c = 0; c < D; ++c) s += DQ[q * D * D + k * D + c] * g[c];
-          sq[k] += s * pj;
+          if constexpr (E::WS) {
+            g[k] = 0.0;
+            for (int r = 0; r < D; ++r) g[k] += JI[q * D * D + k * D + r] * DPHI[(q * NN + i) * D + r];
+          } else {
+            g[k] = GR[(q * NN + i) * D + k];
+          }
+        }
+        for (int k = 0; k < D; ++k) {
+          dg[k] = 0.0;
+          for (int c = 0; c < D; ++c) dg[k] += DQ[q * D * D + k * D + c] * g[c];
           bg += BQ[q * D + k] * g[k];
         }
-        suu += (RQ[q] * pi - bg) * pj;
-      }
-      for (int f = 0; f < NF; ++f) {
-        const int ai = pos[f * NN + i], bj = pos[f * NN + j];
-        if (ai >= 0 && bj >= 0) {
-          const double* F0 = FM + (f * NS) * NNF * NNF + ai * NNF + bj;
-          suu += F0[0];
-          for (int k = 0; k < D; ++k) sq[k] -= F0[(2 + D + k) * NNF * NNF];
+        const double rb = RQ[q] * pi - bg;
+#pragma unroll
+        for (int u = 0; u < JB; ++u) {
+          const double pj = w * PHI[q * NN + ju[u]];
+          m[u] += pi * pj;
+          for (int k = 0; k < D; ++k) {
+            cg[u][k] += g[k] * pj;
+            sq[u][k] += dg[k] * pj;
+          }
+          suu[u] += rb * pj;
         }
       }
-      AUG1[i * NC1 + j] = m;
-      for (int k = 0; k < D; ++k) {
-        AUG1[i * NC1 + NN + k * NN + j] = cg[k];
-        SUQ[(k * NN + i) * NN + j] = sq[k];
+#pragma unroll
+      for (int u = 0; u < JB; ++u) {
+        if (j0 + u * JG >= NN) continue;
+        const int j = ju[u];
+        for (int f = 0; f < NF; ++f) {
+          const int ai = pos[f * NN + i], bj = pos[f * NN + j];
+          if (ai >= 0 && bj >= 0) {
+            const double* F0 = FM + (f * NS) * NNF * NNF + ai * NNF + bj;
+            suu[u] += F0[0];
+            for (int k = 0; k < D; ++k) sq[u][k] -= F0[(2 + D + k) * NNF * NNF];
+          }
+        }
+        AUG1[i * NC1 + j] = m[u];
+        for (int k = 0; k < D; ++k) {
+          AUG1[i * NC1 + NN + k * NN + j] = cg[u][k];
+          SUQ[(k * NN + i) * NN + j] = sq[u][k];
+        }
+        AUG1[i * NC1 + NN + D * NN + j] = (i == j) ? 1.0 : 0.0;
+        SUU[i * NN + j] = suu[u];
       }
-      AUG1[i * NC1 + NN + D * NN + j] = (i == j) ? 1.0 : 0.0;
-      SUU[i * NN + j] = suu;
     }
     for (int i = tid; i < NN; i += NT) {
       double s = 0.0;
+#pragma unroll 4
       for (int q = 0; q < NIP; ++q) s += DV[q] * FQ[q] * PHI[q * NN + i];
       FU[i] = s;
     }
@@ -335,6 +429,7 @@ __global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
       const double* uo = a.u_old + (size_t)e * NN;
       for (int i = tid; i < NN; i += NT) {
         double c = 0.0, mu = 0.0;
+#pragma unroll 4
         for (int j = 0; j < NN; ++j) {
           c += SUU[i * NN + j] * w[j];
           mu += AUG1[i * NC1 + j] * uo[j];
@@ -343,6 +438,7 @@ __global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
         for (int f = 0; f < NF; ++f) {
           const int ai = pos[f * NN + i];
           if (ai < 0) continue;
+#pragma unroll 4
           for (int b = 0; b < NNF; ++b)
             c += (-FM[((f * NS + 0) * NNF + ai) * NNF + b] + FM[((f * NS + 1) * NNF + ai) * NNF + b]) *
                  w[NN * (D + 1) + f * NNF + b];
@@ -403,55 +499,86 @@ __global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
     }
 
     // ---------------------------------- [M | Cg | I] -> [I | A | M^-1]
-    gauss_jordan<NN, NC1, NT>(AUG1, perm1);
+    if constexpr (E::WS && !E::BOTH) gauss_jordan_via<NN, NC1, NT>(AUG1, lds_ws, perm1);
+    else gauss_jordan<NN, NC1, NT>(AUG1, perm1);
     // K = Suu - sum_k Suq_k A_k ;  Z_k = Suq_k M^-1
     for (int t = tid; t < NN * NN; t += NT) {
       const int i = t / NN, j = t % NN;
       double s = SUU[t];
-      for (int k = 0; k < D; ++k)
-        for (int l = 0; l < NN; ++l) s -= SUQ[(k * NN + i) * NN + l] * AUG1[perm1[l] * NC1 + NN + k * NN + j];
+      for (int k = 0; k < D; ++k) {
+        double z = 0.0;
+#pragma unroll 4
+        for (int l = 0; l < NN; ++l) {
+          const double sq = SUQ[(k * NN + i) * NN + l];
+          const double* row = AUG1 + perm1[l] * NC1 + NN;
+          s -= sq * row[k * NN + j];
+          z += sq * row[D * NN + j];
+        }
+        ZB[k * NN * NN + t] = z;
+      }
       AUG2[i * NC2 + j] = s;
     }
-    for (int t = tid; t < D * NN * NN; t += NT) {
-      const int k = t / (NN * NN), i = (t / NN) % NN, j = t % NN;
-      double s = 0.0;
-      for (int l = 0; l < NN; ++l) s += SUQ[(k * NN + i) * NN + l] * AUG1[perm1[l] * NC1 + NN + D * NN + j];
-      ZB[t] = s;
-    }
     __syncthreads();
-    // -R = -(Sul - sum_k Z_k Sql_k) ; Fu
-    for (int t = tid; t < NN * NL; t += NT) {
-      const int i = t / NL, c = t % NL, f = c / NNF, b = c % NNF;
-      double r = 0.0;
-      const int ai = pos[f * NN + i];
-      if (ai >= 0) r = a.ts_arest * (-FM[((f * NS + 0) * NNF + ai) * NNF + b] + FM[((f * NS + 1) * NNF + ai) * NNF + b]);
+    // -R = -(Sul - sum_k Z_k Sql_k) ; Fu.  IB rows per thread share the face masses.
+    constexpr int IB = 4, IG = (NN + IB - 1) / IB;
+    for (int t = tid; t < IG * NL; t += NT) {
+      const int i0 = t / NL, c = t % NL, f = c / NNF, b = c % NNF;
+      int iu[IB];
+      double r[IB];
+#pragma unroll
+      for (int u = 0; u < IB; ++u) {
+        const int i = i0 + u * IG;
+        iu[u] = i < NN ? i : NN - 1;
+        r[u] = 0.0;
+        const int ai = pos[f * NN + iu[u]];
+        if (ai >= 0) r[u] = a.ts_arest * (-FM[((f * NS + 0) * NNF + ai) * NNF + b] + FM[((f * NS + 1) * NNF + ai) * NNF + b]);
+      }
       for (int k = 0; k < D; ++k)
-        for (int aa = 0; aa < NNF; ++aa)
-          r += ZB[(k * NN + i) * NN + fn[f * NNF + aa]] * FM[((f * NS + 2 + k) * NNF + aa) * NNF + b];
-      AUG2[i * NC2 + NN + c] = -r;
+#pragma unroll 4
+        for (int aa = 0; aa < NNF; ++aa) {
+          const double fm = FM[((f * NS + 2 + k) * NNF + aa) * NNF + b];
+          const double* z = ZB + k * NN * NN + fn[f * NNF + aa];
+#pragma unroll
+          for (int u = 0; u < IB; ++u) r[u] += z[iu[u] * NN] * fm;
+        }
+#pragma unroll
+      for (int u = 0; u < IB; ++u)
+        if (i0 + u * IG < NN) AUG2[iu[u] * NC2 + NN + c] = -r[u];
     }
     for (int i = tid; i < NN; i += NT) AUG2[i * NC2 + NN + NL] = FU[i];
     __syncthreads();
     // ---------------------------------------- [K | -R | Fu] -> [I | U | U0]
-    gauss_jordan<NN, NC2, NT>(AUG2, perm2);
+    if constexpr (E::WS && !E::BOTH) gauss_jordan_via<NN, NC2, NT>(AUG2, lds_ws, perm2);
+    else gauss_jordan<NN, NC2, NT>(AUG2, perm2);
     // Q_k = -A_k U - M^-1 Sql_k ;  Q0_k = -A_k U0 ; write U, U0, Q, Q0
     double* Ue = a.U + (size_t)e * NN * NL;
     double* Qe = a.Q + (size_t)e * NN * D * NL;
     for (int t = tid; t < NN * NL; t += NT) Ue[t] = AUG2[perm2[t / NL] * NC2 + NN + t % NL];
     for (int t = tid; t < NN; t += NT) a.U0[(size_t)e * NN + t] = AUG2[perm2[t] * NC2 + NN + NL];
-    for (int t = tid; t < D * NN * NL; t += NT) {
-      const int k = t / (NN * NL), i = (t / NL) % NN, c = t % NL, f = c / NNF, b = c % NNF;
-      double s = 0.0;
-      const int pi = perm1[i];
-      for (int j = 0; j < NN; ++j) s -= AUG1[pi * NC1 + NN + k * NN + j] * AUG2[perm2[j] * NC2 + NN + c];
-      for (int aa = 0; aa < NNF; ++aa)
-        s += AUG1[pi * NC1 + NN + D * NN + fn[f * NNF + aa]] * FM[((f * NS + 2 + k) * NNF + aa) * NNF + b];
-      QL[t] = s;
-      Qe[(size_t)(i * D + k) * NL + c] = s;
+    for (int t = tid; t < NN * NL; t += NT) {
+      const int i = t / NL, c = t % NL, f = c / NNF, b = c % NNF;
+      double s[D];
+      for (int k = 0; k < D; ++k) s[k] = 0.0;
+      const double* row = AUG1 + perm1[i] * NC1 + NN;
+#pragma unroll 4
+      for (int j = 0; j < NN; ++j) {
+        const double uj = AUG2[perm2[j] * NC2 + NN + c];
+        for (int k = 0; k < D; ++k) s[k] -= row[k * NN + j] * uj;
+      }
+#pragma unroll 4
+      for (int aa = 0; aa < NNF; ++aa) {
+        const double mi = row[D * NN + fn[f * NNF + aa]];
+        for (int k = 0; k < D; ++k) s[k] += mi * FM[((f * NS + 2 + k) * NNF + aa) * NNF + b];
+      }
+      for (int k = 0; k < D; ++k) {
+        if constexpr (!E::WS) QL[k * NN * NL + t] = s[k];
+        Qe[(size_t)(i * D + k) * NL + c] = s[k];
+      }
     }
     for (int t = tid; t < D * NN; t += NT) {
       const int k = t / NN, i = t % NN;
       double s = 0.0;
+#pragma unroll 4
       for (int j = 0; j < NN; ++j) s -= AUG1[perm1[i] * NC1 + NN + k * NN + j] * AUG2[perm2[j] * NC2 + NN + NL];
       Q0L[t] = s;
       a.Q0[(size_t)e * NN * D + i * D + k] = s;
@@ -460,23 +587,42 @@ __global__ __launch_bounds__(NT) void hdg_element_kernel(ElemArgs a) {
     // S = Slu U + sum_k Slq_k Q_k + Sll ; S0 = -Slu U0 - sum_k Slq_k Q0_k
     // (explicit HDG modes: S = Sll, S0 = -Slu sol_old - Slq flux_old)
     double* Se = a.S + (size_t)e * NL * NL;
-    for (int t = tid; t < NL * NL; t += NT) {
-      const int r = t / NL, c = t % NL, f = r / NNF, aa = r % NNF;
-      double s = 0.0;
+    constexpr int RB = 3, RG = (NNF + RB - 1) / RB;  // RB rows of a face per thread share U and Q
+    for (int t = tid; t < NF * RG * NL; t += NT) {
+      const int c = t % NL, f = t / (RG * NL), a0 = (t / NL) % RG;
+      int au[RB];
+      double s[RB];
+#pragma unroll
+      for (int u = 0; u < RB; ++u) {
+        au[u] = a0 + u * RG < NNF ? a0 + u * RG : NNF - 1;
+        s[u] = 0.0;
+      }
+#pragma unroll 4
       for (int b = 0; b < NNF && !a.hdg_explicit; ++b) {
         const int j = fn[f * NNF + b];
-        s += FM[((f * NS + 0) * NNF + aa) * NNF + b] * AUG2[perm2[j] * NC2 + NN + c];
-        for (int k = 0; k < D; ++k) s -= FM[((f * NS + 2 + D + k) * NNF + aa) * NNF + b] * QL[(k * NN + j) * NL + c];
+        const double uj = AUG2[perm2[j] * NC2 + NN + c];
+        double qj[D];
+        for (int k = 0; k < D; ++k) qj[k] = E::WS ? Qe[(size_t)(j * D + k) * NL + c] : QL[(k * NN + j) * NL + c];
+#pragma unroll
+        for (int u = 0; u < RB; ++u) {
+          s[u] += FM[((f * NS + 0) * NNF + au[u]) * NNF + b] * uj;
+          for (int k = 0; k < D; ++k) s[u] -= FM[((f * NS + 2 + D + k) * NNF + au[u]) * NNF + b] * qj[k];
+        }
       }
-      if (c / NNF == f) {
-        const int b = c % NNF;
-        s += -FM[((f * NS + 0) * NNF + aa) * NNF + b] + FM[((f * NS + 1) * NNF + aa) * NNF + b];
+#pragma unroll
+      for (int u = 0; u < RB; ++u) {
+        if (a0 + u * RG >= NNF) continue;
+        if (c / NNF == f) {
+          const int b = c % NNF;
+          s[u] += -FM[((f * NS + 0) * NNF + au[u]) * NNF + b] + FM[((f * NS + 1) * NNF + au[u]) * NNF + b];
+        }
+        Se[(f * NNF + au[u]) * NL + c] = s[u];
       }
-      Se[t] = s;
     }
     for (int r = tid; r < NL; r += NT) {
       const int f = r / NNF, aa = r % NNF;
       double s = 0.0;
+#pragma unroll 4
       for (int b = 0; b < NNF; ++b) {
         const int j = fn[f * NNF + b];
         const double uj = a.hdg_explicit ? a.sol_old[(size_t)e * NN + j] : AUG2[perm2[j] * NC2 + NN + NL];
@@ -513,10 +659,10 @@ template <int D, int P, int NT>
 void launch_t(const ElemArgs& a, int grid_cap, hipStream_t s) {
   using L = Layout<D, P, NT>;
   constexpr bool gws = element_in_workspace<D, P>();
-  const size_t lds = gws ? 0 : (size_t)L::TOTAL * sizeof(double);
+  const size_t lds = ElemLds<D, P>::BYTES;
   auto kern = hdg_element_kernel<D, P, NT>;
   static PerDeviceLaunch once;
-  if (!gws) once.lds_attr((const void*)kern, lds);
+  once.lds_attr((const void*)kern, lds);
   int grid = a.nEl;
   if (grid_cap > 0 && grid > grid_cap) grid = grid_cap;
   if (gws) {
