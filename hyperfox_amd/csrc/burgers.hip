@@ -76,28 +76,38 @@ struct BLay {
   static constexpr int O_TAU = O_VN + NN * NV * D;  // [f][j][t]
   static constexpr int O_SOL = O_TAU + NL * MM;  // [i][a]
   static constexpr int O_TR = O_SOL + MU;        // [f][j][a]
-  static constexpr int O_FIP = O_TR + ML;        // [q][a]
+  // The face blocks of tau lie over the gathered inputs, the weighted face
+  // blocks and the solution in row order over [Suq | Slq | ..], each once the
+  // arrays below them are no longer needed.
+  static constexpr int NFB = NF * MM * NNF * NNF, NXU = MU * (ML + 1);
+  static constexpr int bmax(int a, int b) { return a > b ? a : b; }
+  static constexpr int O_FT = O_X;               // [f][t][a][b] sum_q dS tau_t psi_a psi_b
+  static constexpr int O_FIP = bmax(O_TR + ML, O_FT + NFB);  // [q][a] source, then the u part of F_u
   static constexpr int O_DV = O_FIP + NIP * M;
   static constexpr int O_GR = O_DV + NIP;        // [q][i][k] physical grad phi_i
-  static constexpr int O_UQ = O_GR + NIP * NN * D;  // [q][a]
-  static constexpr int O_DIV = O_UQ + NIP * M;
+  static constexpr int O_UQ = O_GR + NIP * NN * D;  // [q][a] dV u_a
+  static constexpr int O_UU = O_UQ + NIP * M;    // [q][a][k] dV u_a u_k (HDGUNabU)
+  static constexpr int O_DIV = O_UU + (MDL == 0 ? NIP * MM : 0);  // dV div u
   static constexpr int O_DQ = O_DIV + NIP;      // [c][q]
-  static constexpr int O_VQ = O_DQ + NDC * NIP;  // [q][t][k]
+  static constexpr int O_VQ = O_DQ + NDC * NIP;  // [q][t][k] dV v_t
   static constexpr int O_FDS = O_VQ + NIP * NV * D;  // [f][q] face measure
   static constexpr int O_FN = O_FDS + NFQ;       // [f][q][k] outward normal
-  static constexpr int O_LAM = O_FN + NFQ * D;   // [f][q][a] trace
-  static constexpr int O_USF = O_LAM + NFQ * M;  // [f][q][a] cell solution
-  static constexpr int O_TQ = O_USF + NFQ * M;   // [f][q][t] tau
-  static constexpr int O_DFQ = O_TQ + NFQ * MM;  // [c][f q]
-  static constexpr int O_VFN = O_DFQ + NDC * NFQ;  // [f q][t] v_t . n
-  static constexpr int O_FL = O_VFN + NFQ * NV;  // F_l [ML]
+  static constexpr int O_FLQ = O_FN + NFQ * D;   // [f][q][a] dS (lambda.n)(lambda_a + u_a)/2
+  static constexpr int O_TQ = O_FLQ + NFQ * M;   // [f][q][t] dS tau_t
+  static constexpr int O_WQ = O_TQ + NFQ * MM;   // [f][q][t] dS times the weight of the face's u/lambda coupling
+  static constexpr int O_DFQ = O_WQ + NFQ * MM;  // [c][f q]
+  static constexpr int O_FL = O_DFQ + NDC * NFQ;  // F_l [ML]
   static constexpr int O_AUG1 = O_FL + ML;
   static constexpr int O_SUQ = O_AUG1 + NN * NC1;          // [c][k][i][j]
   static constexpr int O_SLQ = O_SUQ + NDC * D * NN * NN;  // [c][k][f nNf + a][j]
   static constexpr int O_KS = O_SLQ + NDC * D * NL * NN;   // [c] sum_k Suq_k A_k
   static constexpr int O_RS = O_KS + NDC * NN * NN;        // [c] sum_k Suq_k B_k
   static constexpr int O_P = O_RS + NDC * NN * NL;         // [c] sum_k Slq_k A_k
-  static constexpr int O_PB = O_P + NDC * NL * NN;         // [c] sum_k Slq_k B_k
+  static constexpr bool FW_OVER = NFB <= NDC * D * (NN * NN + NL * NN);
+  static constexpr int O_XU = O_SUQ + (FW_OVER ? NFB : 0);  // [r][l] U and U0, from the end of Slu's assembly
+  static constexpr int O_XE = bmax(O_P + NDC * NL * NN, O_XU + NXU);
+  static constexpr int O_FW = FW_OVER ? O_SUQ : O_XE;  // [f][t][a][b] the blocks of WQ, from the end of Suq's use
+  static constexpr int O_PB = O_XE + (FW_OVER ? 0 : NFB);  // [c] sum_k Slq_k B_k
   static constexpr int O_SLU = O_PB + NDC * NL * NL;       // Slu - P (x) I  [ML][MU]
   static constexpr int O_AUG2 = O_SLU + ML * MU;
   static constexpr int TOTAL = O_AUG2 + MU * NC2;
@@ -126,6 +136,17 @@ constexpr bool burgers_in_workspace() {
   return (size_t)BLay<D, P, MDL>::TOTAL * sizeof(double) > 150 * 1024;
 }
 
+// Bound by the chain of its phases (a gather of dependent loads, a dozen
+// barriers, 30 elimination steps), which the workgroups of a CU cover for each
+// other, and by the LDS reads of the sums.  So the index chains of the gather
+// run on different wavefronts; whatever a face or a cubature point contributes
+// to several blocks is formed once (the face blocks of tau and of the coupling
+// weights enter K, R, Slu and Sll); a thread takes all components of a node
+// pair, so that each value read serves several sums; and the grid is what the
+// device holds at once, so that the tables are read once per workgroup.
+// Measured, 18,432 2-D p=3 Burgers cells: 2.09 ms before, 1.08 ms (1.66 ms with
+// the shorter elimination alone).  Recomputing the index arithmetic for every
+// cell instead of keeping it in registers (no spills) took 1.26 ms.
 template <int D, int P, int MDL>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(burgers_waves<D, P, MDL>())))
 void burgers_cell_kernel(BurgersArgs a) {
@@ -178,12 +199,11 @@ void burgers_cell_kernel(BurgersArgs a) {
   double* DQ = sm + L::O_DQ;
   double* VN = sm + L::O_VN;
   double* VQ = sm + L::O_VQ;
-  double* VFN = sm + L::O_VFN;
   double* FDS = sm + L::O_FDS;
   double* FN = sm + L::O_FN;
-  double* LAM = sm + L::O_LAM;
-  double* USF = sm + L::O_USF;
+  double* FLQ = sm + L::O_FLQ;
   double* TQ = sm + L::O_TQ;
+  double* WQ = sm + L::O_WQ;
   double* DFQ = sm + L::O_DFQ;
   double* FL = sm + L::O_FL;
   double* AUG1 = sm + L::O_AUG1;
@@ -194,6 +214,10 @@ void burgers_cell_kernel(BurgersArgs a) {
   double* PP = sm + L::O_P;
   double* PB = sm + L::O_PB;
   double* SLU = sm + L::O_SLU;
+  double* UU = sm + L::O_UU;
+  double* FT = sm + L::O_FT;
+  double* FWB = sm + L::O_FW;
+  double* XU = sm + L::O_XU;
   double* AUG2 = sm + L::O_AUG2;
   // coefficient set c of component a: cs_of(a); set c present: has_c(c)
   auto cs_of = [](int comp) { return MDL == 1 ? comp : 0; };
@@ -201,22 +225,24 @@ void burgers_cell_kernel(BurgersArgs a) {
 
   for (int e = blockIdx.x; e < a.nEl; e += gridDim.x) {
     __syncthreads();  // the previous cell's outputs are written
-    // ------------------------------------------------------------ gather
+    // ------------------------------------------------------------ gather,
+    // each chain of dependent loads on wavefronts of its own
+    auto from_wave = [&](int w) { return (tid + BT - 64 * w) & (BT - 1); };
     for (int t = tid; t < NN * D; t += BT) X[t] = a.coords[(size_t)a.cells[(size_t)e * NN + t / D] * D + t % D];
-    for (int t = tid; t < NDC * NN; t += BT) {
+    for (int t = from_wave(1); t < NDC * NN; t += BT) {
       const int c = t / NN, node = a.cells[(size_t)e * NN + t % NN];
       const double* src = c == 0 ? a.Dn : a.G;
       DN[t] = src ? src[node] : 0.0;
     }
-    for (int t = tid; t < NL * MM; t += BT) {
+    for (int t = from_wave(2); t < NL * MM; t += BT) {
       const int fj = t / MM, c = t % MM, f = fj / NNF;
       const int F = a.cell2face[(size_t)e * NF + f];
       const int side = (a.tau_sides == 2 && a.face2cell[2 * (size_t)F] != e) ? 1 : 0;
       const int p = a.face_perm[(size_t)e * NL + fj];
       TAU[t] = a.tau[(((size_t)F * NNF + p) * a.tau_sides + side) * MM + c];
     }
-    for (int t = tid; t < MU; t += BT) SOL[t] = a.sol[(size_t)e * MU + t];
-    for (int t = tid; t < ML; t += BT) {
+    for (int t = from_wave(1); t < MU; t += BT) SOL[t] = a.sol[(size_t)e * MU + t];
+    for (int t = from_wave(3); t < ML; t += BT) {
       const int fj = t / M, f = fj / NNF;
       const int F = a.cell2face[(size_t)e * NF + f];
       TR[t] = a.trace[((size_t)F * NNF + a.face_perm[(size_t)e * NL + fj]) * M + t % M];
@@ -226,6 +252,7 @@ void burgers_cell_kernel(BurgersArgs a) {
       if (a.u_old && a.ts_idt != 0.0) {  // implicit Euler: + u_old(x_q) / dt
         const int q = t / M, c = t % M;
         double uo = 0.0;
+#pragma unroll 4
         for (int j = 0; j < NN; ++j) uo += PHI[q * NN + j] * a.u_old[((size_t)e * NN + j) * M + c];
         fq += a.ts_idt * uo;
       }
@@ -250,6 +277,7 @@ void burgers_cell_kernel(BurgersArgs a) {
     for (int q = tid; q < NIP; q += BT) {
       double J[D * D];
       for (int t = 0; t < D * D; ++t) J[t] = 0.0;
+#pragma unroll 2
       for (int i = 0; i < NN; ++i)
         for (int r = 0; r < D; ++r)
           for (int c = 0; c < D; ++c) J[r * D + c] += DPHI[(q * NN + i) * D + r] * X[i * D + c];
@@ -260,6 +288,7 @@ void burgers_cell_kernel(BurgersArgs a) {
       double uq[D], dv = 0.0, dq[NDC];
       for (int c = 0; c < NDC; ++c) dq[c] = 0.0;
       for (int c = 0; c < M; ++c) uq[c] = 0.0;
+#pragma unroll 2
       for (int i = 0; i < NN; ++i) {
         const double ph = PHI[q * NN + i];
         for (int k = 0; k < D; ++k) {
@@ -271,19 +300,27 @@ void burgers_cell_kernel(BurgersArgs a) {
         for (int c = 0; c < M; ++c) uq[c] += ph * SOL[i * M + c];
         for (int c = 0; c < NDC; ++c) dq[c] += ph * DN[c * NN + i];
       }
-      for (int c = 0; c < M; ++c) UQ[q * M + c] = uq[c];
-      DIV[q] = dv;
+      const double wd = DV[q];
+      for (int c = 0; c < M; ++c) {
+        UQ[q * M + c] = wd * uq[c];
+        FIP[q * M + c] = wd * (MDL == 0 ? FIP[q * M + c] - uq[c] * dv : FIP[q * M + c]);
+        if constexpr (MDL == 0)
+          for (int k = 0; k < D; ++k) UU[(q * M + c) * D + k] = wd * uq[c] * uq[k];
+      }
+      DIV[q] = wd * dv;
       for (int c = 0; c < NDC; ++c) DQ[c * NIP + q] = dq[c];
       for (int tk = 0; tk < NV * D; ++tk) {
         double v = 0.0;
+#pragma unroll 2
         for (int i = 0; i < NN; ++i) v += PHI[q * NN + i] * VN[i * NV * D + tk];
-        VQ[q * NV * D + tk] = v;
+        VQ[q * NV * D + tk] = wd * v;
       }
     }
     for (int t = tid; t < NFQ; t += BT) {
       const int f = t / NIPF, q = t % NIPF;
       double Jf[(D - 1) * D];
       for (int u = 0; u < (D - 1) * D; ++u) Jf[u] = 0.0;
+#pragma unroll 4
       for (int j = 0; j < NNF; ++j) {
         const double* xj = X + fn[f * NNF + j] * D;
         for (int r = 0; r < D - 1; ++r)
@@ -322,6 +359,7 @@ void burgers_cell_kernel(BurgersArgs a) {
       for (int c = 0; c < NDC; ++c) dfq[c] = 0.0;
       for (int c = 0; c < M; ++c) lam[c] = us[c] = 0.0;
       for (int c = 0; c < MM; ++c) tq[c] = 0.0;
+#pragma unroll 4
       for (int j = 0; j < NNF; ++j) {
         const double ps = FPHI[q * NNF + j];
         const int nj = fn[f * NNF + j];
@@ -332,21 +370,29 @@ void burgers_cell_kernel(BurgersArgs a) {
         for (int c = 0; c < MM; ++c) tq[c] += ps * TAU[(f * NNF + j) * MM + c];
         for (int c = 0; c < NDC; ++c) dfq[c] += ps * DN[c * NN + nj];
       }
-      for (int c = 0; c < M; ++c) {
-        LAM[t * M + c] = lam[c];
-        USF[t * M + c] = us[c];
-      }
-      for (int c = 0; c < MM; ++c) TQ[t * MM + c] = tq[c];
       for (int c = 0; c < NDC; ++c) DFQ[c * NFQ + t] = dfq[c];
-      for (int tv = 0; tv < NV; ++tv) {
-        double vn = 0.0;
-        for (int k = 0; k < D; ++k) {
-          double v = 0.0;
-          for (int j = 0; j < NNF; ++j) v += FPHI[q * NNF + j] * VN[(fn[f * NNF + j] * NV + tv) * D + k];
-          vn += v * nv[k];
+      const double ds = FDS[t];
+      double ln = 0.0;
+      if constexpr (MDL == 0)
+        for (int k = 0; k < D; ++k) ln += lam[k] * nv[k];
+      for (int c = 0; c < M; ++c) FLQ[t * M + c] = ds * 0.5 * ln * (lam[c] + us[c]);
+      for (int na = 0; na < M; ++na)
+        for (int mb = 0; mb < M; ++mb) {
+          double w = -tq[mb * M + na];
+          if constexpr (MDL == 0) {  // HDGUNabU face rows
+            w += us[na] * nv[mb];
+            if (na == mb) w += ln;
+          } else if constexpr (MDL == 1) {  // HDGConvection: (v.n) face mass
+            for (int k = 0; k < D; ++k) {
+              double v = 0.0;
+#pragma unroll 4
+              for (int j = 0; j < NNF; ++j) v += FPHI[q * NNF + j] * VN[(fn[f * NNF + j] * NV + na * M + mb) * D + k];
+              w += v * nv[k];
+            }
+          }
+          TQ[t * MM + na * M + mb] = ds * tq[na * M + mb];
+          WQ[t * MM + na * M + mb] = ds * w;
         }
-        VFN[t * (NV > 0 ? NV : 1) + tv] = vn;
-      }
     }
     __syncthreads();
     // ------------------------------------------------ scalar q blocks
@@ -354,14 +400,17 @@ void burgers_cell_kernel(BurgersArgs a) {
       const int i = t / NC1, c = t % NC1;
       double v = 0.0;
       if (c < NN) {
+#pragma unroll 4
         for (int q = 0; q < NIP; ++q) v += DV[q] * PHI[q * NN + i] * PHI[q * NN + c];
       } else if (c < NN + D * NN) {
         const int k = (c - NN) / NN, j = (c - NN) % NN;
+#pragma unroll 4
         for (int q = 0; q < NIP; ++q) v += DV[q] * GR[(q * NN + i) * D + k] * PHI[q * NN + j];
       } else {
         const int cc = c - NN - D * NN, k = cc / NL, fc = cc % NL, f = fc / NNF, cn = fc % NNF;
         const int ai = posf[f * NN + i];
         if (ai >= 0)
+#pragma unroll 4
           for (int q = 0; q < NIPF; ++q) {
             const int o = f * NIPF + q;
             v -= FDS[o] * FN[o * D + k] * FPHI[q * NNF + ai] * FPHI[q * NNF + cn];
@@ -375,10 +424,12 @@ void burgers_cell_kernel(BurgersArgs a) {
       const double* dfc = DFQ + c * NFQ;
       double v = 0.0;
       if (has_c(c)) {
+#pragma unroll 4
         for (int q = 0; q < NIP; ++q) v += DV[q] * dqc[q] * GR[(q * NN + i) * D + k] * PHI[q * NN + j];
         for (int f = 0; f < NF; ++f) {
           const int ai = posf[f * NN + i], cj = posf[f * NN + j];
           if (ai < 0 || cj < 0) continue;
+#pragma unroll 4
           for (int q = 0; q < NIPF; ++q) {
             const int o = f * NIPF + q;
             v -= FDS[o] * dfc[o] * FN[o * D + k] * FPHI[q * NNF + ai] * FPHI[q * NNF + cj];
@@ -394,12 +445,21 @@ void burgers_cell_kernel(BurgersArgs a) {
       const double* dfc = DFQ + c * NFQ;
       double v = 0.0;
       if (has_c(c) && cj >= 0)
+#pragma unroll 4
         for (int q = 0; q < NIPF; ++q) {
           const int o = f * NIPF + q;
           v -= FDS[o] * dfc[o] * FN[o * D + k] * FPHI[q * NNF + ai] * FPHI[q * NNF + cj];
         }
       SLQ[t] = v;
     }
+    auto face_block = [&](const double* wq, int t) {  // t = [f][t][a][b]
+      const int f = t / (MM * NNF * NNF), c = (t / (NNF * NNF)) % MM, ai = (t / NNF) % NNF, b = t % NNF;
+      double v = 0.0;
+#pragma unroll 4
+      for (int q = 0; q < NIPF; ++q) v += wq[(f * NIPF + q) * MM + c] * FPHI[q * NNF + ai] * FPHI[q * NNF + b];
+      return v;
+    };
+    for (int t = tid; t < L::NFB; t += BT) FT[t] = face_block(TQ, t);
     __syncthreads();
     gauss_jordan<NN, NC1, BT>(AUG1, perm1);
     // A_k[i][j] = AUG1[perm1[i] NC1 + NN + k NN + j], B_k[i][fc] = AUG1[perm1[i] NC1 + NN + D NN + k NL + fc]
@@ -425,6 +485,7 @@ void burgers_cell_kernel(BurgersArgs a) {
       }
       double v = 0.0;
       for (int k = 0; k < D; ++k)
+#pragma unroll 4
         for (int l = 0; l < NN; ++l) {
           const double* xr = AUG1 + perm1[l] * NC1 + NN + (isA ? k * NN : D * NN + k * NL);
           v += Lrow[k * ncol + l] * xr[col];
@@ -432,114 +493,88 @@ void burgers_cell_kernel(BurgersArgs a) {
       *dst = v;
     }
     __syncthreads();
+    for (int t = tid; t < L::NFB; t += BT) FWB[t] = face_block(WQ, t);
+    __syncthreads();
     // ----------------------------------- coupled blocks [K | R | F_u], Slu, F_l
-    for (int t = tid; t < MU * NC2; t += BT) {
-      const int r = t / NC2, c = t % NC2, i = r / M, na = r % M;
-      double v = 0.0;
-      if (c < MU) {
-        const int j = c / M, mb = c % M;
-        for (int f = 0; f < NF; ++f) {  // HDGBase tau
-          const int ai = posf[f * NN + i], cj = posf[f * NN + j];
-          if (ai < 0 || cj < 0) continue;
-          for (int q = 0; q < NIPF; ++q) {
-            const int o = f * NIPF + q;
-            v += FDS[o] * TQ[o * MM + mb * M + na] * FPHI[q * NNF + ai] * FPHI[q * NNF + cj];
-          }
+    auto fb = [](const double* b, int f, int c, int ai, int cn) { return b[((f * MM + c) * NNF + ai) * NNF + cn]; };
+    for (int t = tid; t < MU * NN; t += BT) {  // K: the M columns of node j together
+      const int r = t / NN, j = t % NN, i = r / M, na = r % M;
+      double acc[M];
+      for (int mb = 0; mb < M; ++mb) acc[mb] = 0.0;
+      for (int f = 0; f < NF; ++f) {  // HDGBase tau
+        const int ai = posf[f * NN + i], cj = posf[f * NN + j];
+        if (ai < 0 || cj < 0) continue;
+        for (int mb = 0; mb < M; ++mb) acc[mb] += fb(FT, f, mb * M + na, ai, cj);
+      }
+      if constexpr (MDL == 0) {
+#pragma unroll 2
+        for (int q = 0; q < NIP; ++q) {  // HDGUNabU bulk
+          const double* gi = GR + (q * NN + i) * D;
+          const double* gj = GR + (q * NN + j) * D;
+          const double pi = PHI[q * NN + i], pj = PHI[q * NN + j], ua = UQ[q * M + na];
+          double ug = DIV[q] * pi;
+          for (int k = 0; k < D; ++k) ug += UQ[q * M + k] * gi[k];
+          for (int mb = 0; mb < M; ++mb) acc[mb] -= ua * (gj[mb] * pi + gi[mb] * pj) + (na == mb ? ug * pj : 0.0);
         }
-        if constexpr (MDL == 0) {
-          for (int q = 0; q < NIP; ++q) {  // HDGUNabU bulk
-            const double* gi = GR + (q * NN + i) * D;
-            const double* gj = GR + (q * NN + j) * D;
-            const double pi = PHI[q * NN + i], pj = PHI[q * NN + j];
-            double w = UQ[q * M + na] * (gj[mb] * pi + gi[mb] * pj);
-            if (na == mb) {
-              double ug = 0.0;
-              for (int k = 0; k < D; ++k) ug += UQ[q * M + k] * gi[k];
-              w += (DIV[q] * pi + ug) * pj;
-            }
-            v -= DV[q] * w;
-          }
-        } else if constexpr (MDL == 1) {
-          for (int q = 0; q < NIP; ++q) {  // HDGConvection of v_(na mb): Suu -= C^T
-            const double* gi = GR + (q * NN + i) * D;
+      } else if constexpr (MDL == 1) {
+#pragma unroll 2
+        for (int q = 0; q < NIP; ++q) {  // HDGConvection of v_(na mb): Suu -= C^T
+          const double* gi = GR + (q * NN + i) * D;
+          const double pj = PHI[q * NN + j];
+          for (int mb = 0; mb < M; ++mb) {
             const double* vq = VQ + (q * NV + na * M + mb) * D;
             double vg = 0.0;
             for (int k = 0; k < D; ++k) vg += vq[k] * gi[k];
-            v -= DV[q] * vg * PHI[q * NN + j];
-          }
-        }
-        if (na == mb) {
-          v -= KS[cs_of(na) * NN * NN + i * NN + j];
-          if (a.ts_idt != 0.0) {  // implicit Euler: + M / dt
-            double mij = 0.0;
-            for (int q = 0; q < NIP; ++q) mij += DV[q] * PHI[q * NN + i] * PHI[q * NN + j];
-            v += a.ts_idt * mij;
-          }
-        }
-      } else if (c < MU + ML) {
-        const int l = c - MU, f = l / (NNF * M), cn = (l / M) % NNF, mb = l % M;
-        const int ai = posf[f * NN + i];
-        if (ai >= 0)
-          for (int q = 0; q < NIPF; ++q) {
-            const int o = f * NIPF + q;
-            double w = -TQ[o * MM + mb * M + na];
-            if constexpr (MDL == 0) {  // HDGUNabU face rows summed into the u rows
-              double ln = 0.0;
-              for (int k = 0; k < D; ++k) ln += LAM[o * M + k] * FN[o * D + k];
-              w += USF[o * M + na] * FN[o * D + mb];
-              if (na == mb) w += ln;
-            } else if constexpr (MDL == 1) {  // HDGConvection: Sul += (v.n) face mass
-              w += VFN[o * (NV > 0 ? NV : 1) + na * M + mb];
-            }
-            v += FDS[o] * w * FPHI[q * NNF + ai] * FPHI[q * NNF + cn];
-          }
-        if (na == mb) v -= RS[cs_of(na) * NN * NL + i * NL + f * NNF + cn];
-        v = -v;
-      } else {
-        for (int q = 0; q < NIP; ++q) {
-          const double* gi = GR + (q * NN + i) * D;
-          double ug = 0.0;
-          for (int k = 0; k < D; ++k) ug += UQ[q * M + k] * gi[k];
-          double w = PHI[q * NN + i] * FIP[q * M + na];
-          if constexpr (MDL == 0) w -= UQ[q * M + na] * (DIV[q] * PHI[q * NN + i] + ug);
-          v += DV[q] * w;
-        }
-        for (int f = 0; f < NF && MDL == 0; ++f) {
-          const int ai = posf[f * NN + i];
-          if (ai < 0) continue;
-          for (int q = 0; q < NIPF; ++q) {
-            const int o = f * NIPF + q;
-            double ln = 0.0;
-            for (int k = 0; k < D; ++k) ln += LAM[o * M + k] * FN[o * D + k];
-            v += FDS[o] * FPHI[q * NNF + ai] * 0.5 * ln * (LAM[o * M + na] + USF[o * M + na]);
+            acc[mb] -= vg * pj;
           }
         }
       }
-      AUG2[t] = v;
+      double mij = 0.0;
+      if (a.ts_idt != 0.0)  // implicit Euler: + M / dt
+#pragma unroll 4
+        for (int q = 0; q < NIP; ++q) mij += DV[q] * PHI[q * NN + i] * PHI[q * NN + j];
+      for (int mb = 0; mb < M; ++mb) {
+        if (na == mb) acc[mb] += a.ts_idt * mij - KS[cs_of(na) * NN * NN + i * NN + j];
+        AUG2[r * NC2 + j * M + mb] = acc[mb];
+      }
     }
-    for (int t = tid; t < ML * MU + ML; t += BT) {
-      if (t < ML * MU) {
-        const int rl = t / MU, c = t % MU, f = rl / (NNF * M), ai = (rl / M) % NNF, na = rl % M;
-        const int j = c / M, mb = c % M, cj = posf[f * NN + j];
-        double v = 0.0;
-        if (cj >= 0)
-          for (int q = 0; q < NIPF; ++q) {
-            const int o = f * NIPF + q;
-            v += FDS[o] * TQ[o * MM + mb * M + na] * FPHI[q * NNF + ai] * FPHI[q * NNF + cj];
-          }
-        if (na == mb) v -= PP[cs_of(na) * NL * NN + (f * NNF + ai) * NN + j];
-        SLU[t] = v;
-      } else {
-        const int rl = t - ML * MU, f = rl / (NNF * M), ai = (rl / M) % NNF, na = rl % M;
-        double v = 0.0;
-        for (int q = 0; q < NIPF && MDL == 0; ++q) {
-          const int o = f * NIPF + q;
-          double ln = 0.0;
-          for (int k = 0; k < D; ++k) ln += LAM[o * M + k] * FN[o * D + k];
-          v += FDS[o] * FPHI[q * NNF + ai] * 0.5 * ln * (LAM[o * M + na] + USF[o * M + na]);
-        }
-        FL[rl] = v;
+    for (int t = tid; t < MU * ML; t += BT) {
+      const int r = t / ML, l = t % ML, i = r / M, na = r % M, f = l / (NNF * M), cn = (l / M) % NNF, mb = l % M;
+      const int ai = posf[f * NN + i];
+      double v = ai >= 0 ? fb(FWB, f, na * M + mb, ai, cn) : 0.0;
+      if (na == mb) v -= RS[cs_of(na) * NN * NL + i * NL + f * NNF + cn];
+      AUG2[r * NC2 + MU + l] = -v;
+    }
+    for (int t = tid; t < ML * MU; t += BT) {
+      const int rl = t / MU, c = t % MU, f = rl / (NNF * M), ai = (rl / M) % NNF, na = rl % M;
+      const int j = c / M, mb = c % M, cj = posf[f * NN + j];
+      double v = cj >= 0 ? fb(FT, f, mb * M + na, ai, cj) : 0.0;
+      if (na == mb) v -= PP[cs_of(na) * NL * NN + (f * NNF + ai) * NN + j];
+      SLU[t] = v;
+    }
+    for (int t = from_wave(3); t < MU; t += BT) {  // F_u
+      const int i = t / M, na = t % M;
+      double v = 0.0;
+#pragma unroll 4
+      for (int q = 0; q < NIP; ++q) {
+        v += PHI[q * NN + i] * FIP[q * M + na];
+        if constexpr (MDL == 0)
+          for (int k = 0; k < D; ++k) v -= GR[(q * NN + i) * D + k] * UU[(q * M + na) * D + k];
       }
+      for (int f = 0; f < NF && MDL == 0; ++f) {
+        const int ai = posf[f * NN + i];
+        if (ai < 0) continue;
+#pragma unroll 4
+        for (int q = 0; q < NIPF; ++q) v += FPHI[q * NNF + ai] * FLQ[(f * NIPF + q) * M + na];
+      }
+      AUG2[t * NC2 + MU + ML] = v;
+    }
+    for (int t = from_wave(2); t < ML; t += BT) {  // F_l
+      const int f = t / (NNF * M), ai = (t / M) % NNF, na = t % M;
+      double v = 0.0;
+#pragma unroll 4
+      for (int q = 0; q < NIPF && MDL == 0; ++q) v += FPHI[q * NNF + ai] * FLQ[(f * NIPF + q) * M + na];
+      FL[t] = v;
     }
     __syncthreads();
     gauss_jordan<MU, NC2, BT>(AUG2, perm2);
@@ -549,51 +584,67 @@ void burgers_cell_kernel(BurgersArgs a) {
     for (int t = tid; t < MU * (ML + 1); t += BT) {
       const int r = t / (ML + 1), l = t % (ML + 1);
       const double v = AUG2[perm2[r] * NC2 + MU + l];
+      XU[t] = v;
       if (l < ML) Ue[(size_t)r * ML + l] = v;
       else a.U0[(size_t)e * MU + r] = v;
     }
-    for (int t = tid; t < D * MU * (ML + 1); t += BT) {
-      const int rq = t / (ML + 1), l = t % (ML + 1);
-      const int i = rq / (D * M), k = (rq / M) % D, na = rq % M;
-      const double* Ak = AUG1 + NN + k * NN;
-      double v = 0.0;
-      for (int j = 0; j < NN; ++j) v -= Ak[perm1[i] * NC1 + j] * AUG2[perm2[j * M + na] * NC2 + MU + l];
-      if (l < ML) {
-        const int fc = l / M, mb = l % M;
-        if (na == mb) v -= AUG1[perm1[i] * NC1 + NN + D * NN + k * NL + fc];
-        Qe[(size_t)rq * ML + l] = v;
-      } else {
-        a.Q0[(size_t)e * D * MU + rq] = v;
+    __syncthreads();
+    for (int t = tid; t < NN * (ML + 1); t += BT) {  // Q, Q0: every (k, component) of node i and column l
+      const int i = t / (ML + 1), l = t % (ML + 1);
+      const double* row = AUG1 + perm1[i] * NC1 + NN;
+      double v[D][M];
+      for (int k = 0; k < D; ++k)
+        for (int na = 0; na < M; ++na) v[k][na] = 0.0;
+#pragma unroll 2
+      for (int j = 0; j < NN; ++j) {
+        double x[M];
+        for (int na = 0; na < M; ++na) x[na] = XU[(j * M + na) * (ML + 1) + l];
+        for (int k = 0; k < D; ++k) {
+          const double ak = row[k * NN + j];
+          for (int na = 0; na < M; ++na) v[k][na] -= ak * x[na];
+        }
       }
-    }
-    for (int t = tid; t < ML * (ML + 1); t += BT) {
-      const int rl = t / (ML + 1), l = t % (ML + 1);
-      const double* sr = SLU + rl * MU;
-      if (l < ML) {
-        double v = 0.0;
-        for (int r = 0; r < MU; ++r) v += sr[r] * AUG2[perm2[r] * NC2 + MU + l];
-        const int f = rl / (NNF * M), ai = (rl / M) % NNF, na = rl % M;
-        const int g = l / (NNF * M), cn = (l / M) % NNF, mb = l % M;
-        if (f == g)
-          for (int q = 0; q < NIPF; ++q) {  // Sll: HDGBase tau and HDGUNabU / HDGConvection face terms
-            const int o = f * NIPF + q;
-            double w = -TQ[o * MM + mb * M + na];
-            if constexpr (MDL == 0) {
-              double ln = 0.0;
-              for (int k = 0; k < D; ++k) ln += LAM[o * M + k] * FN[o * D + k];
-              w += USF[o * M + na] * FN[o * D + mb];
-              if (na == mb) w += ln;
-            } else if constexpr (MDL == 1) {
-              w += VFN[o * (NV > 0 ? NV : 1) + na * M + mb];
-            }
-            v += FDS[o] * w * FPHI[q * NNF + ai] * FPHI[q * NNF + cn];
+      for (int k = 0; k < D; ++k)
+        for (int na = 0; na < M; ++na) {
+          const int rq = (i * D + k) * M + na;
+          if (l < ML) {
+            if (na == l % M) v[k][na] -= row[D * NN + k * NL + l / M];
+            Qe[(size_t)rq * ML + l] = v[k][na];
+          } else {
+            a.Q0[(size_t)e * D * MU + rq] = v[k][na];
           }
-        if (na == mb) v -= PB[cs_of(na) * NL * NL + (f * NNF + ai) * NL + g * NNF + cn];
-        a.S[((size_t)e * ML + rl) * ML + l] = v;
+        }
+    }
+    for (int t = tid; t < NL * (NL + 1); t += BT) {  // S, S0: the M x M block of two face nodes
+      const int fa = t / (NL + 1), g = t % (NL + 1), f = fa / NNF, ai = fa % NNF;
+      const double* sr = SLU + fa * M * MU;
+      if (g < NL) {
+        double v[M][M];
+        for (int na = 0; na < M; ++na)
+          for (int mb = 0; mb < M; ++mb) v[na][mb] = 0.0;
+#pragma unroll 2
+        for (int r = 0; r < MU; ++r) {
+          double x[M];
+          for (int mb = 0; mb < M; ++mb) x[mb] = XU[r * (ML + 1) + g * M + mb];
+          for (int na = 0; na < M; ++na) {
+            const double sv = sr[na * MU + r];
+            for (int mb = 0; mb < M; ++mb) v[na][mb] += sv * x[mb];
+          }
+        }
+        for (int na = 0; na < M; ++na)
+          for (int mb = 0; mb < M; ++mb) {
+            double w = v[na][mb];
+            if (f == g / NNF) w += fb(FWB, f, na * M + mb, ai, g % NNF);  // Sll
+            if (na == mb) w -= PB[cs_of(na) * NL * NL + fa * NL + g];
+            a.S[((size_t)e * ML + fa * M + na) * ML + g * M + mb] = w;
+          }
       } else {
-        double v = FL[rl];
-        for (int r = 0; r < MU; ++r) v -= sr[r] * AUG2[perm2[r] * NC2 + MU + ML];
-        a.S0[(size_t)e * ML + rl] = v;
+        for (int na = 0; na < M; ++na) {
+          double v = FL[fa * M + na];
+#pragma unroll 4
+          for (int r = 0; r < MU; ++r) v -= sr[na * MU + r] * XU[r * (ML + 1) + ML];
+          a.S0[(size_t)e * ML + fa * M + na] = v;
+        }
       }
     }
   }
@@ -605,7 +656,9 @@ void launch_dp(const BurgersArgs& a, hipStream_t s) {
   const size_t lds = gws ? 0 : (size_t)BLay<D, P, MDL>::TOTAL * sizeof(double);
   static PerDeviceLaunch once;
   if (!gws) once.lds_attr((const void*)burgers_cell_kernel<D, P, MDL>, lds);
-  int grid = a.nEl < 65536 ? a.nEl : 65536;
+  // as many workgroups as the device holds at once: each reads the tables once
+  const long long cap = once.resident_wgs((const void*)burgers_cell_kernel<D, P, MDL>, BT, lds);
+  int grid = (int)(a.nEl < cap ? a.nEl : cap);
   if (gws) {
     if (!a.gws || a.gws_slots <= 0) throw std::runtime_error("Burgers kernel: this order needs its device workspace");
     if (grid > a.gws_slots) grid = a.gws_slots;
