@@ -921,6 +921,14 @@ constexpr int INLINE_PARTIALS = 2048;
 // L2, about the time of the extra launch); longer ones reduce them first.
 constexpr int GM_INLINE = 128;
 
+// Above this many blocks the steps are bound by memory and not by the chain of
+// one block, and few rows in registers (more wavefronts) beat one read of the
+// basis: chunks of 8 rows in the product (which reads them once either way),
+// of 16 in the orthogonalisation.  GMRES(30) on 1.69 M rows of 10 x 10 blocks:
+// 232 ms with chunks of 32, 193 ms (227 ms before the four-launch steps); on
+// 0.5 M rows (2,000 blocks) chunks of 32 take 61 ms, 64 ms before.
+constexpr int GM_TALL = 4096;
+
 void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
             hipStream_t s, KrylovWs* kws) {
   const long long n = A.nrows();
@@ -955,6 +963,7 @@ void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const
   }
   const double target = o.rtol * bnorm;
   KrylovStatus* st = hw.host();
+  const bool tall = nblk > GM_TALL;
   const bool inl = nblk <= GM_INLINE, inl3 = nblk <= INLINE_PARTIALS;
   const int tiles = M.kind == PC_BJACOBI ? ceil_div(n, (RT / A.bs) * A.bs) : nblk;
   double* sums3 = inl3 ? p3 : gs + GM_NORM2 + 1;  // ||w||^2
@@ -983,7 +992,7 @@ void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const
 #define HFX_LAUNCH(B, KC)                                                                                           \
   hipLaunchKernelGGL((gm_product_kernel<B, KC>), dim3(grid), dim3(RT), 0, s, A.nb, A.rowptr.p, A.col.p, A.vals.p, z, \
                      w, k, V, (long long)ln, nblk, p1, target, seq, gs, st)
-#define HFX_BS(B) case B: if (k <= 8) HFX_LAUNCH(B, 8); else if (k <= 16) HFX_LAUNCH(B, 16); else HFX_LAUNCH(B, 32); break;
+#define HFX_BS(B) case B: if (k <= 8 || tall) HFX_LAUNCH(B, 8); else if (k <= 16) HFX_LAUNCH(B, 16); else HFX_LAUNCH(B, 32); break;
     switch (A.bs) {
       HFX_BS(1) HFX_BS(2) HFX_BS(3) HFX_BS(4) HFX_BS(5) HFX_BS(6) HFX_BS(7) HFX_BS(8) HFX_BS(9) HFX_BS(10) HFX_BS(11) HFX_BS(12) HFX_BS(15) HFX_BS(18) HFX_BS(21) HFX_BS(30)
       default: throw std::runtime_error("spmv: unsupported block size");
@@ -1025,7 +1034,7 @@ void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const
 #define HFX_LAUNCH(KC)                                                                                              \
   hipLaunchKernelGGL((gm_orth_kernel<KC>), dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h1, w, nblk, p2, gs)
       if (k <= 8) HFX_LAUNCH(8);
-      else if (k <= 16) HFX_LAUNCH(16);
+      else if (k <= 16 || tall) HFX_LAUNCH(16);
       else HFX_LAUNCH(32);
 #undef HFX_LAUNCH
       HFX_HIP(hipGetLastError());
