@@ -623,13 +623,15 @@ __device__ __forceinline__ void block_sums(double* v, int c0, int k, double* __r
 
 // w = A z (thread per row) with the partials of V_i . w, i < k, in
 // partial[i nblk + blk]; block nblk finishes Hessenberg column k - 2.
-template <int BS, int KC>
+// Chunks of KC basis rows: eight, at every size (see gm_orth_kernel).
+template <int BS>
 __global__ __launch_bounds__(RT) void gm_product_kernel(int nb, const int* __restrict__ rowptr,
                                                         const int* __restrict__ col, const double* __restrict__ vals,
                                                         const double* __restrict__ z, double* __restrict__ w, int k,
                                                         const double* __restrict__ V, long long ldv, int nblk,
                                                         double* __restrict__ partial, double target, int seq,
                                                         double* gs, KrylovStatus* st) {
+  constexpr int KC = 8;
   __shared__ double red[RT / 64][KC];
   if (gm_flag(gs, GM_SEEN)) return;
   if ((int)blockIdx.x == nblk) {
@@ -685,7 +687,14 @@ __device__ __forceinline__ void gather_h(int k, int np, const double* __restrict
 }
 
 // w -= V h, then the partials of V_i . w: the V values of a row stay in
-// registers between the two (up to KC of them)
+// registers between the two (up to KC of them; from KC on they are read again).
+// Few rows in registers, and so more wavefronts, beat one read of the basis:
+// with chunks of 8 in the product and 8 (k <= 8) or 16 here, 126 steps take, in
+// ms at restart 30 / 63 (in brackets with chunks of 32 from k = 17 on),
+//      37 blocks  3.9 / 5.2 (3.9 / 5.4)     340 blocks   4.4 /  6.6 (5.1 /  8.2)
+//   1,333 blocks 13.3 / 18.5 (16.0 / 26.1)  3,391 blocks 20.7 / 32.5 (27.7 / 52.1)
+// (block sizes 3, 2, 10 and 2, block Jacobi), the larger two 20.7 / 26.8 and
+// 23.6 / 36.0 before the four-launch steps.  The order of every sum is the same.
 template <int KC>
 __global__ __launch_bounds__(RT) void gm_orth_kernel(long long n, int k, const double* __restrict__ V, long long ldv,
                                                      int np, const double* __restrict__ part, double* __restrict__ w,
@@ -921,14 +930,6 @@ constexpr int INLINE_PARTIALS = 2048;
 // L2, about the time of the extra launch); longer ones reduce them first.
 constexpr int GM_INLINE = 128;
 
-// Above this many blocks the steps are bound by memory and not by the chain of
-// one block, and few rows in registers (more wavefronts) beat one read of the
-// basis: chunks of 8 rows in the product (which reads them once either way),
-// of 16 in the orthogonalisation.  GMRES(30) on 1.69 M rows of 10 x 10 blocks:
-// 232 ms with chunks of 32, 193 ms (227 ms before the four-launch steps); on
-// 0.5 M rows (2,000 blocks) chunks of 32 take 61 ms, 64 ms before.
-constexpr int GM_TALL = 4096;
-
 void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,
             hipStream_t s, KrylovWs* kws) {
   const long long n = A.nrows();
@@ -963,7 +964,6 @@ void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const
   }
   const double target = o.rtol * bnorm;
   KrylovStatus* st = hw.host();
-  const bool tall = nblk > GM_TALL;
   const bool inl = nblk <= GM_INLINE, inl3 = nblk <= INLINE_PARTIALS;
   const int tiles = M.kind == PC_BJACOBI ? ceil_div(n, (RT / A.bs) * A.bs) : nblk;
   double* sums3 = inl3 ? p3 : gs + GM_NORM2 + 1;  // ||w||^2
@@ -989,16 +989,16 @@ void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const
   auto product = [&](int j, int seq) {
     const int k = j + 1, grid = nblk + (j > 0 ? 1 : 0);
     const double* z = Z + (size_t)j * ln;
-#define HFX_LAUNCH(B, KC)                                                                                           \
-  hipLaunchKernelGGL((gm_product_kernel<B, KC>), dim3(grid), dim3(RT), 0, s, A.nb, A.rowptr.p, A.col.p, A.vals.p, z, \
-                     w, k, V, (long long)ln, nblk, p1, target, seq, gs, st)
-#define HFX_BS(B) case B: if (k <= 8 || tall) HFX_LAUNCH(B, 8); else if (k <= 16) HFX_LAUNCH(B, 16); else HFX_LAUNCH(B, 32); break;
+#define HFX_BS(B)                                                                                                   \
+  case B:                                                                                                           \
+    hipLaunchKernelGGL((gm_product_kernel<B>), dim3(grid), dim3(RT), 0, s, A.nb, A.rowptr.p, A.col.p, A.vals.p, z,  \
+                       w, k, V, (long long)ln, nblk, p1, target, seq, gs, st);                                      \
+    break;
     switch (A.bs) {
       HFX_BS(1) HFX_BS(2) HFX_BS(3) HFX_BS(4) HFX_BS(5) HFX_BS(6) HFX_BS(7) HFX_BS(8) HFX_BS(9) HFX_BS(10) HFX_BS(11) HFX_BS(12) HFX_BS(15) HFX_BS(18) HFX_BS(21) HFX_BS(30)
       default: throw std::runtime_error("spmv: unsupported block size");
     }
 #undef HFX_BS
-#undef HFX_LAUNCH
     HFX_HIP(hipGetLastError());
   };
   // the partials of V^T w, or (long vectors) their sums
@@ -1034,8 +1034,7 @@ void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const
 #define HFX_LAUNCH(KC)                                                                                              \
   hipLaunchKernelGGL((gm_orth_kernel<KC>), dim3(nblk), dim3(RT), 0, s, n, k, V, (long long)ln, nph, h1, w, nblk, p2, gs)
       if (k <= 8) HFX_LAUNCH(8);
-      else if (k <= 16 || tall) HFX_LAUNCH(16);
-      else HFX_LAUNCH(32);
+      else HFX_LAUNCH(16);
 #undef HFX_LAUNCH
       HFX_HIP(hipGetLastError());
       const double* h2 = rows(k, p2, hr + 64);

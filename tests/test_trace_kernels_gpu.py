@@ -111,6 +111,32 @@ def test_gmres_against_a_dense_solve(n, restart):
         assert la.last_info[:2] == (its - 1, -3) and la.last_info[2] > 1e-11
 
 
+@pytest.mark.parametrize('restart', [8, 9, 16, 17, 24, 33, 63])
+def test_gmres_cycles_longer_than_a_chunk(restart):
+    """Cycles that end on either side of a chunk of basis rows (8 in the product, 8 or 16 in the orthogonalisation) and
+    run through several of them, on a five-point Laplacian that needs more steps than a cycle has."""
+    print('gmres long', restart, flush=True)
+    n = 40
+    T = 2.0 * np.eye(n) - np.eye(n, k=1) - np.eye(n, k=-1)
+    A = np.kron(T, np.eye(n)) + np.kron(np.eye(n), T) + np.diag(1e-5 * np.arange(n * n))
+    b = np.random.default_rng(5).standard_normal(n * n)
+    la = hf.HipLinAlgebra(hf.HipOpts(rtol=1e-10, maxits=5000, restart=restart))
+    la.initialize()
+    la.configure()
+    la.allocate(n * n)
+    for i in range(n * n):
+        cols = np.nonzero(A[i])[0]
+        la.setValsMatrix([i], cols, A[i, cols])
+    la.setValsRHS(np.arange(n * n), b)
+    la.assemble()
+    x = np.array(la.solve())
+    its, reason, rel = la.last_info
+    assert its > restart  # a whole cycle ran
+    assert reason == 2 and rel <= 1e-10
+    ref = np.linalg.solve(A, b)
+    assert np.linalg.norm(x - ref) <= np.linalg.cond(A) * 1e-10 * np.linalg.norm(ref)
+
+
 @pytest.mark.parametrize('ordering', [hf.linalg.PC_ILU0, hf.linalg.PC_ILU0_NATURAL], ids=['multicolour', 'natural'])
 @pytest.mark.parametrize('pattern', ['diagonal', 'one-way', 'lower', 'chain', 'dense'])
 def test_ilu_sweeps_on_odd_patterns(pattern, ordering):
