@@ -137,6 +137,53 @@ def test_gmres_cycles_longer_than_a_chunk(restart):
     assert np.linalg.norm(x - ref) <= np.linalg.cond(A) * 1e-10 * np.linalg.norm(ref)
 
 
+def host_gmres(A, dinv, b, m, steps):
+    """Right-preconditioned GMRES(m) from zero for `steps` steps, Gram-Schmidt twice; the iterate."""
+    x, done = np.zeros_like(b), 0
+    while done < steps:
+        k = min(m, steps - done)
+        r = b - A @ x
+        beta = np.linalg.norm(r)
+        V, H = np.zeros((k + 1, b.size)), np.zeros((k + 1, k))
+        V[0] = r / beta
+        for j in range(k):
+            w = A @ (dinv * V[j])
+            for _ in range(2):
+                h = V[:j + 1] @ w
+                w -= h @ V[:j + 1]
+                H[:j + 1, j] += h
+            H[j + 1, j] = np.linalg.norm(w)
+            V[j + 1] = w / H[j + 1, j]
+        y = np.linalg.lstsq(H, beta * np.eye(k + 1)[0], rcond=None)[0]
+        x += dinv * (y @ V[:k])
+        done += k
+    return x
+
+
+@pytest.mark.parametrize('n,restart,steps', [(73, 30, 34), (75, 30, 34), (75, 63, 45), (294, 12, 14), (298, 30, 34),
+                                             (298, 63, 45)])
+def test_gmres_on_long_vectors(n, restart, steps):
+    """Row blocks (256 rows) on both sides of the sizes where the sums over the blocks are reduced by a kernel of their
+    own: V^T w above 128 (n = 73: 127, 75: 134), ||w||^2 too above 2,048 (n = 294: 2,031, 298: 2,086); cycles of more
+    than 32 columns, and a step budget that ends inside a cycle.  The residual that the solver reports is the one of
+    the solution it returns, and is the least that so many steps can reach, as found on the host: the residual of a
+    GMRES iterate is within a small multiple of k^(3/2) eps (|| |A| |x| || + ||b||) of that."""
+    print('gmres long vectors', n, restart, steps, flush=True)
+    import scipy.sparse as sp
+    w, prob = problem(2, 1, n)
+    prob.set_krylov(hf.KRYLOV_FGMRES)
+    its, reason, rel = prob.solve(pc=hf.PC_JACOBI, rtol=1e-14, maxits=steps, restart=restart)
+    assert (its, reason) == (steps, -3)
+    rowptr, cols, vals, b = prob.trace_csr()
+    A = sp.csr_matrix((vals, cols, rowptr))
+    x = prob.solution()[2]
+    nb = np.linalg.norm(b)
+    eps = EPS * (np.linalg.norm(abs(A) @ np.abs(x)) + nb) / nb
+    assert abs(np.linalg.norm(b - A @ x) / nb - rel) <= 8 * eps
+    ref = host_gmres(A, 1.0 / A.diagonal(), b, restart, steps)
+    assert abs(np.linalg.norm(b - A @ ref) / nb - rel) <= 8 * steps ** 1.5 * eps
+
+
 @pytest.mark.parametrize('ordering', [hf.linalg.PC_ILU0, hf.linalg.PC_ILU0_NATURAL], ids=['multicolour', 'natural'])
 @pytest.mark.parametrize('pattern', ['diagonal', 'one-way', 'lower', 'chain', 'dense'])
 def test_ilu_sweeps_on_odd_patterns(pattern, ordering):
