@@ -92,8 +92,8 @@ struct ElemArgs {
   int hdg_explicit = 0;
   const double* sol_old = nullptr;
   const double* flux_old = nullptr;
-  // orders whose element working set exceeds the LDS (3-D p = 4, 5): a
-  // device workspace of element_workspace_doubles() doubles per workgroup,
+  // orders whose element working set exceeds the LDS (2-D p >= 7, 3-D
+  // p = 4, 5): a device workspace of element_workspace_doubles() doubles per workgroup,
   // gws_slots of them; the grid is capped at gws_slots
   double* gws = nullptr;
   int gws_slots = 0;
@@ -103,8 +103,9 @@ struct ElemArgs {
 // a.el_offset; `nt` threads per element (64, 128 or 256).  Throws on error.
 void launch_element(int dim, int order, const ElemArgs& a, int nt, int grid_cap, hipStream_t s);
 
-// Dynamic LDS bytes the kernel needs for (dim, order): 0 for the orders
-// that keep the element's working set in a device workspace instead.
+// Dynamic LDS bytes the kernel needs for (dim, order): the element's working
+// set, or its elimination matrices for the orders that keep the rest in a
+// device workspace.
 size_t element_lds_bytes(int dim, int order);
 // Doubles of device workspace per workgroup for (dim, order); 0 when the
 // working set is in LDS.

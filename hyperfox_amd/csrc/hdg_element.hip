@@ -687,9 +687,8 @@ void launch_dp(const ElemArgs& a, int nt, int grid_cap, hipStream_t s) {
 }  // namespace
 
 size_t element_lds_bytes(int dim, int order) {
-#define HFX_CASE(D, P)                                                                             \
-  if (dim == D && order == P)                                                                      \
-    return element_in_workspace<D, P>() ? 0 : (size_t)Layout<D, P, 64>::TOTAL * sizeof(double);
+#define HFX_CASE(D, P) \
+  if (dim == D && order == P) return ElemLds<D, P>::BYTES;
   HFX_CASE(2, 1) HFX_CASE(2, 2) HFX_CASE(2, 3) HFX_CASE(2, 4) HFX_CASE(2, 5)
   HFX_CASE(2, 6) HFX_CASE(2, 7) HFX_CASE(2, 8) HFX_CASE(2, 9) HFX_CASE(2, 10)
   HFX_CASE(3, 1) HFX_CASE(3, 2) HFX_CASE(3, 3) HFX_CASE(3, 4) HFX_CASE(3, 5)

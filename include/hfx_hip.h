@@ -329,10 +329,11 @@ int hfx_hdg_get_solution(hfx_hdg* h, double* u, double* q, double* lambda);
  * 2 trace solve with the last solve's options.  ms receives `reps` values. */
 int hfx_hdg_time(hfx_hdg* h, int what, int warmup, int reps, double* ms);
 
-/* Dynamic LDS bytes used by the general element kernel of (dim, order); 0
- * for the orders (3-D p = 4, 5) whose element working set does not fit the
- * LDS and lives in a device workspace instead (hfx_element_workspace_bytes).
- * The reference supports 2-D p <= 10 and 3-D p <= 5
+/* Dynamic LDS bytes used by the general element kernel of (dim, order).  The
+ * orders whose element working set does not fit the LDS (2-D p >= 7, 3-D
+ * p >= 4) keep it in a device workspace (hfx_element_workspace_bytes) except
+ * for the matrices of the two eliminations: both (3-D p = 4, 2-D p <= 9) or
+ * the one at work are in LDS.  The reference supports 2-D p <= 10 and 3-D p <= 5
  * (ReferenceElement.cpp:620-623), and so does the GPU path (2-D p >= 7 and
  * 3-D p >= 4 in the device workspace). */
 int hfx_element_lds_bytes(int dim, int order, long long* bytes);

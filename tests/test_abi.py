@@ -46,8 +46,12 @@ def test_unsupported_gpu_orders_rejected_before_any_device_call():
 def test_high_orders_keep_the_element_in_a_device_workspace(dim, p):
     # 3-D p = 4, 5 and 2-D p >= 7 (ReferenceElement.cpp:620-623): the
     # element's working set exceeds the 160 KB of LDS, so the kernel takes a
-    # per-workgroup slab of device memory instead (2-D p = 6 still fits)
+    # per-workgroup slab of device memory (2-D p = 6 still fits) and keeps in
+    # LDS an elimination matrix: [M | Cg | I] or [K | R | F], the larger, or both
     v = ctypes.c_longlong()
-    assert hf.lib.hfx_element_lds_bytes(dim, p, ctypes.byref(v)) == 0 and v.value == 0
+    s = hf.refel_sizes(dim, p)
+    m1, m2 = 8 * s['nN'] * s['nN'] * (dim + 2), 8 * s['nN'] * (s['nN'] + s['lenL'] + 1)
+    assert hf.lib.hfx_element_lds_bytes(dim, p, ctypes.byref(v)) == 0
+    assert max(m1, m2) <= v.value <= min(m1 + m2, 160 * 1024)
     assert hf.lib.hfx_element_workspace_bytes(dim, p, ctypes.byref(v)) == 0 and v.value > 160 * 1024
     assert hf.lib.hfx_element_lds_bytes(2, 6, ctypes.byref(v)) == 0 and 0 < v.value <= 160 * 1024
