@@ -180,7 +180,6 @@ hfx::PcApply make_pc(hfx_burgers* h, int pc) {
     hfx::bsr_inv_point_diag(h->A, h->dinv.p, s);
     M.kind = hfx::PC_JACOBI;
     M.dinv = h->dinv.p;
-    M.fn = [h, n, s](const double* in, double* out) { hfx::apply_point_diag(n, h->dinv.p, in, out, s); };
     return M;
   }
   if (pc == HFX_PC_BJACOBI) {
@@ -188,7 +187,6 @@ hfx::PcApply make_pc(hfx_burgers* h, int pc) {
     hfx::bsr_invert_diag(h->A, h->dinv.p, s);
     M.kind = hfx::PC_BJACOBI;
     M.dinv = h->dinv.p;
-    M.fn = [h, s](const double* in, double* out) { hfx::apply_block_diag(h->A.nb, h->A.bs, h->dinv.p, in, out, s); };
     return M;
   }
   if (pc == HFX_PC_ILU0 || pc == HFX_PC_ILU0_F32) {

@@ -345,11 +345,8 @@ extern "C" int hfx_la_solve(hfx_la* h, double* x, int n, int* info, double* relr
     HFX_HIP(hipMemsetAsync(h->dx.p, 0, (size_t)h->n * sizeof(double), s));
     hfx::PcApply M;
     if (h->pc == HFX_PC_JACOBI) {
-      const double* dinv = h->dinv.p;
-      const long long nn = h->n;
       M.kind = hfx::PC_JACOBI;
-      M.dinv = dinv;
-      M.fn = [dinv, nn, s](const double* in, double* out) { hfx::apply_point_diag(nn, dinv, in, out, s); };
+      M.dinv = h->dinv.p;
     } else if (h->pc == HFX_PC_ILU0 || h->pc == HFX_PC_ILU0_NATURAL) {
       const int ord = h->pc == HFX_PC_ILU0 ? hfx::ILU_MULTICOLOUR : hfx::ILU_NATURAL;
       if (h->ilu_stale || !h->ilu || h->ilu->ordering != ord) {

@@ -657,7 +657,6 @@ __global__ void ip_coords_kernel(int nEl, const double* __restrict__ tabs, const
 
 template <int D, int P, int NT>
 void launch_t(const ElemArgs& a, int grid_cap, hipStream_t s) {
-  using L = Layout<D, P, NT>;
   constexpr bool gws = element_in_workspace<D, P>();
   const size_t lds = ElemLds<D, P>::BYTES;
   auto kern = hdg_element_kernel<D, P, NT>;

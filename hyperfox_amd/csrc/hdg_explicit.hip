@@ -69,8 +69,8 @@ struct XLay {
   static constexpr int O_FO = O_SO + NN;
   static constexpr int O_FG = O_FO + NN * D;           // per face: n, measure
   static constexpr int O_SV = O_FG + NF * (D + 1);     // [q] s, v in the reference frame
-  static constexpr int O_FT = O_SV + NIP * (D + 1);    // face points: dS tau, dS (b.n - tau), h, S0 integrand
-  static constexpr int O_FU = O_FT + 4 * NFP;
+  static constexpr int O_FT = O_SV + NIP * (D + 1);    // face points: dS (b.n - tau), h, S0 integrand
+  static constexpr int O_FU = O_FT + 3 * NFP;
   static constexpr int O_U0 = O_FU + NN;
   static constexpr int O_Y = O_U0 + NN;                // Ahat_a U0
   static constexpr int PER = (O_Y + D * NN + 1) & ~1;
@@ -225,10 +225,9 @@ __global__ __launch_bounds__(64 * XW) void hdg_explicit_stage_kernel(ElemArgs a)
         }
       }
       const double ds = FWQ[p] * n[D];
-      FT[t] = ds * tq;
-      FT[NFP + t] = ds * (bn - tq);
-      FT[2 * NFP + t] = ds * (tq * (wl - wu) + d * wn - bn * wl);
-      FT[3 * NFP + t] = ds * (d * qn - tq * us);
+      FT[t] = ds * (bn - tq);
+      FT[NFP + t] = ds * (tq * (wl - wu) + d * wn - bn * wl);
+      FT[2 * NFP + t] = ds * (d * qn - tq * us);
     }
     wave_sync();
     // ------------------------------------------------------- F and U0, Q0
@@ -243,7 +242,7 @@ __global__ __launch_bounds__(64 * XW) void hdg_explicit_stage_kernel(ElemArgs a)
         const int j = s_pos[f * NN + i];
         if (j < 0) continue;
         #pragma unroll 4
-        for (int p = 0; p < NIPF; ++p) s += FT[2 * NFP + f * NIPF + p] * FPHI[p * NNF + j];
+        for (int p = 0; p < NIPF; ++p) s += FT[NFP + f * NIPF + p] * FPHI[p * NNF + j];
       }
       FU[i] = s;
     }
@@ -275,14 +274,14 @@ __global__ __launch_bounds__(64 * XW) void hdg_explicit_stage_kernel(ElemArgs a)
       const int f = t / NNF, j = t % NNF;
       double s = 0.0;
       #pragma unroll 4
-      for (int p = 0; p < NIPF; ++p) s += FT[3 * NFP + f * NIPF + p] * FPHI[p * NNF + j];
+      for (int p = 0; p < NIPF; ++p) s += FT[2 * NFP + f * NIPF + p] * FPHI[p * NNF + j];
       a.S0[(size_t)e * NL + t] = s;
     }
     for (int t = lane; t < NF * NNF * NNF; t += 64) {
       const int f = t / (NNF * NNF), i = (t / NNF) % NNF, j = t % NNF;
       double s = 0.0;
       #pragma unroll 4
-      for (int p = 0; p < NIPF; ++p) s += FT[NFP + f * NIPF + p] * (FPHI[p * NNF + i] * FPHI[p * NNF + j]);
+      for (int p = 0; p < NIPF; ++p) s += FT[f * NIPF + p] * (FPHI[p * NNF + i] * FPHI[p * NNF + j]);
       if constexpr (FUSED) {
         const int F = a.cell2face[(size_t)e * NF + f], side = a.face2cell[2 * (size_t)F] == e ? 0 : 1;
         const int8_t* pm = a.face_perm + (size_t)e * NL + f * NNF;

@@ -17,9 +17,9 @@ namespace hfx {
 
 enum PcType { PC_NONE = 0, PC_JACOBI = 1, PC_BJACOBI = 2, PC_OTHER = 3 };
 
-// A preconditioner set up on the matrix: fn(in, out) applies it (empty for
-// PC_NONE).  The solvers fuse point and block Jacobi into the vector kernel
-// before them and read dinv themselves.
+// A preconditioner set up on the matrix.  The solvers fuse point and block
+// Jacobi into the vector kernel before them and read dinv themselves; they call
+// fn(in, out) only for PC_OTHER.
 struct PcApply {
   PcType kind = PC_NONE;
   const double* dinv = nullptr;  // PC_JACOBI: n values, PC_BJACOBI: bs x bs row-major blocks
@@ -83,20 +83,18 @@ void bsr_inv_point_diag(const BsrDev& A, double* dinv, hipStream_t s);
 void apply_block_diag(int nb, int bs, const double* dinv, const double* x, double* y, hipStream_t s);
 void apply_point_diag(long long n, const double* dinv, const double* x, double* y, hipStream_t s);
 
-// Deterministic FP64 dot / norm helpers (two-stage reductions).  The
-// partials live in buffers of its own (init(n)) or in caller memory of
-// Reducer::doubles(n) values (init(n, mem)).
+// Deterministic FP64 norm (two-stage reduction).  The partials live in buffers
+// of its own (init(n)) or in caller memory of Reducer::doubles(n) values
+// (init(n, mem)), where BiCGStab keeps the partials of its x/r update too.
 struct Reducer {
   DevBuf<double> partial_buf, out_buf;
-  double* partial = nullptr;  // grid * 66
-  double* out = nullptr;      // 132
+  double* partial = nullptr;  // grid (caller memory: grid * 66)
+  double* out = nullptr;
   int grid = 0;
   static int grid_for(long long n);
   static size_t doubles(long long n) { return (size_t)grid_for(n) * 66 + 132; }
   void init(long long n);
   void init(long long n, double* mem);
-  // out[j] = V_j . w for j < k (V column-major, leading dim ldv); result on device in out.p
-  void multidot(long long n, int k, const double* V, long long ldv, const double* w, hipStream_t s);
   double norm(long long n, const double* x, hipStream_t s);  // synchronous
 };
 

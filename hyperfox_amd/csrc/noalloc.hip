@@ -98,12 +98,10 @@ extern "C" int hfx_hdg_solve_noalloc(hfx_hdg* h, int pc, double rtol, int maxits
       hfx::bsr_inv_point_diag(A, dinv, s);
       M.kind = hfx::PC_JACOBI;
       M.dinv = dinv;
-      M.fn = [n, dinv, s](const double* in, double* out) { hfx::apply_point_diag(n, dinv, in, out, s); };
     } else if (pc == HFX_PC_BJACOBI) {
       hfx::bsr_invert_diag(A, dinv, s);
       M.kind = hfx::PC_BJACOBI;
       M.dinv = dinv;
-      M.fn = [&A, dinv, s](const double* in, double* out) { hfx::apply_block_diag(A.nb, A.bs, dinv, in, out, s); };
     }
     HFX_HIP(hipMemsetAsync(h->lambda.p, 0, n * sizeof(double), s));  // zero initial guess, as PETSc
     hfx::KrylovOpts o;
