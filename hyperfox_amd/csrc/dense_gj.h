@@ -4,29 +4,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include "wave.h"
+
 namespace hfx {
 
-// value of v in another lane of the row of 16 (DPP control CTRL)
-template <int CTRL>
-__device__ __forceinline__ double gj_dpp(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-
-__device__ __forceinline__ double gj_lane(double v, int l) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
-}
-
-// largest v of the wavefront, the same value in every lane: butterflies inside
-// each row of 16 lanes (quad_perm, row_half_mirror, row_mirror), then one value
-// of each row
+// largest v of the wavefront, the same value in every lane
 __device__ __forceinline__ double gj_wave_max(double v) {
-  v = fmax(v, gj_dpp<0xB1>(v));
-  v = fmax(v, gj_dpp<0x4E>(v));
-  v = fmax(v, gj_dpp<0x141>(v));
-  v = fmax(v, gj_dpp<0x140>(v));
-  return fmax(fmax(gj_lane(v, 0), gj_lane(v, 16)), fmax(gj_lane(v, 32), gj_lane(v, 48)));
+  v = row_max(v);
+  return fmax(fmax(lane_value(v, 0), lane_value(v, 16)), fmax(lane_value(v, 32), lane_value(v, 48)));
 }
 
 // Gauss-Jordan elimination with partial pivoting, without row swaps, on an

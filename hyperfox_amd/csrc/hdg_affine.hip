@@ -22,6 +22,7 @@
 // the only workgroup barrier is the one after the reference tables are staged.
 #include "hdg_element.h"
 #include "hfx_internal.h"
+#include "wave.h"
 
 namespace hfx {
 
@@ -33,12 +34,6 @@ namespace {
 
 typedef double dvec4 __attribute__((ext_vector_type(4)));
 typedef double dvec2 __attribute__((ext_vector_type(2)));
-
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Scheduling hint for a fully unrolled block of NM MFMAs fed by ND LDS
 // reads: alternate one MFMA with its share of the reads and a few VALU
@@ -64,13 +59,6 @@ __device__ inline double recip(double x) {
   r = fma(r, e, r);
   e = fma(-x, r, 1.0);
   return fma(r, e, r);
-}
-
-// value of v in lane l (l uniform across the wave)
-__device__ inline double readlane_d(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-  return __hiloint2double(hi, lo);
 }
 
 template <int D, int P, bool TD>
@@ -743,12 +731,12 @@ __device__ __forceinline__ void affine_cells(const ElemArgs& a, int e_first, int
         const int p = __builtin_amdgcn_readfirstlane(dpp_argmax(fabs(kr[k]), cand));
         used |= 1ull << p;
         const bool elim = cand && lane != p;
-        const double rp = recip(readlane_d(kr[k], p));
+        const double rp = recip(lane_value(kr[k], p));
         myk = lane == p ? k : myk;
         myrd = lane == p ? rp : myrd;
         const double l = elim ? kr[k] * rp : 0.0;
 #pragma unroll
-        for (int j = k + 1; j < NN; ++j) kr[j] = fma(-l, readlane_d(kr[j], p), kr[j]);
+        for (int j = k + 1; j < NN; ++j) kr[j] = fma(-l, lane_value(kr[j], p), kr[j]);
         kr[k] = elim ? l : kr[k];
       }
       // stored column by column, KM[j * NN + k] = LU[k][j]: a substitution

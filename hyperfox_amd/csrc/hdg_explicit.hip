@@ -22,6 +22,7 @@
 // there: 4.41 ms with the full condensation, 1.19 ms (2.7 TB/s).
 #include "hdg_element.h"
 #include "hfx_internal.h"
+#include "wave.h"
 
 namespace hfx {
 
@@ -30,12 +31,6 @@ struct RefConst;
 #include "data/refel_const.inc"
 
 namespace {
-
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Wavefronts (cells) per workgroup: they share the tables (36 KB at 3-D p=3),
 // so 16 of them fit where two workgroups of 4 would.  Measured at the size

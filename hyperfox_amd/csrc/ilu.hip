@@ -4,8 +4,8 @@
 #include <string>
 
 #include "bsr_row.h"
-#include "dense_gj.h"
 #include "ilu.h"
+#include "wave.h"
 
 #include <algorithm>
 
@@ -100,10 +100,7 @@ __global__ __launch_bounds__(FT) void ilu_factor_kernel(const int* __restrict__ 
       v = fabs(M[t * bs + c]);
       if (v != v) v = -1.0;
     }
-    double top = fmax(v, gj_dpp<0xB1>(v));
-    top = fmax(top, gj_dpp<0x4E>(top));
-    top = fmax(top, gj_dpp<0x141>(top));
-    top = gj_lane(fmax(top, gj_dpp<0x140>(top)), 0);
+    const double top = lane_value(row_max(v), 0);
     const int idx = __ffsll(__ballot(v == top)) - 1;
     const int p = (dc != dc) ? c : idx;
     const double best = (dc != dc) ? dc : top;

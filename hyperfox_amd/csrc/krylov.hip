@@ -4,6 +4,7 @@
 
 #include "bsr_row.h"
 #include "krylov.h"
+#include "wave.h"
 
 namespace hfx {
 
@@ -11,23 +12,16 @@ namespace {
 
 constexpr int RT = 256;  // reduction block size
 
-// value of v, CTRL & 15 lanes to the right in its row of 16 (DPP row_shl)
-template <int CTRL>
-__device__ __forceinline__ double row_shl(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true);
-  return __hiloint2double(hi, lo);
-}
-
 // sum over the wavefront, valid in lane 0: the tree of lane distances 32, 16,
-// 8, .., 1, the steps inside a row of 16 lanes as DPP moves
+// 8, .., 1, the steps inside a row of 16 lanes as
+// DPP moves (row_shl)
 __device__ __forceinline__ double wave_sum(double v) {
   v += __shfl_down(v, 32, 64);
   v += __shfl_down(v, 16, 64);
-  v += row_shl<0x108>(v);
-  v += row_shl<0x104>(v);
-  v += row_shl<0x102>(v);
-  v += row_shl<0x101>(v);
+  v += dpp_move<0x108, true>(v);
+  v += dpp_move<0x104, true>(v);
+  v += dpp_move<0x102, true>(v);
+  v += dpp_move<0x101, true>(v);
   return v;
 }
 
@@ -58,12 +52,6 @@ __global__ void spmv_kernel(int nb, const int* __restrict__ rowptr, const int* _
   const int F = (int)(t / BS), r = (int)(t % BS);
   const double acc = bsr_row_sum<BS>(rowptr[F], rowptr[F + 1], r, col, vals, x);
   y[t] = b ? b[t] - acc : acc;
-}
-
-__device__ __forceinline__ void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Inverses of the diagonal blocks by Gauss-Jordan with partial pivoting: one
@@ -103,7 +91,7 @@ __global__ __launch_bounds__(64 * IW) void invert_diag_kernel(int nb, const int*
       const double v = fabs(a[k]);
       col[r] = used ? -2.0 : (v >= 0.0 ? v : -1.0);
     }
-    wave_fence();
+    wave_sync();
     int p = 0;
     double best = col[0];
 #pragma unroll
@@ -125,14 +113,14 @@ __global__ __launch_bounds__(64 * IW) void invert_diag_kernel(int nb, const int*
         perm[k] = r;
       }
     }
-    wave_fence();
+    wave_sync();
     if (!piv) {
       const double f = a[k];
 #pragma unroll
       for (int c = 0; c < BS; ++c) a[c] = c == k ? -f * row[c] : fma(-f, row[c], a[c]);
     }
   }
-  wave_fence();
+  wave_sync();
   if (on) {
     double* dst = dinv + ((size_t)F * BS + myk) * BS;
 #pragma unroll
@@ -485,12 +473,6 @@ enum { GM_DONE = 0, GM_COLS = 1, GM_SEEN = 2 };  // ints at gs + GM_FLAGS
 
 __device__ __forceinline__ int gm_flag(const double* gs, int which) {
   return reinterpret_cast<const int*>(gs + GM_FLAGS)[which];
-}
-
-__device__ __forceinline__ double lane_value(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-  return __hiloint2double(hi, lo);
 }
 
 // Finish column c of the Hessenberg matrix (h1 + h2 and the norm): apply the

@@ -4,6 +4,7 @@
 #include <stdexcept>
 
 #include "trace_system.h"
+#include "wave.h"
 
 namespace hfx {
 
@@ -291,9 +292,7 @@ __global__ __launch_bounds__(64 * RWAVES) void reconstruct_kernel(
       const int f = t / bs;
       L[t] = lambda[(size_t)cell2face[(size_t)e * nFpc + f] * bs + face_perm[(size_t)e * NL + t]];
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();
     const double* Ue = U + (size_t)e * nN * NL;
     const double* Qe = Q + (size_t)e * nQ * NL;
     for (int r0 = 0; r0 < rows; r0 += NR * RPP) {
@@ -323,9 +322,7 @@ __global__ __launch_bounds__(64 * RWAVES) void reconstruct_kernel(
         }
       }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // L is reused by the next cell
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();  // L is reused by the next cell
   }
 }
 
