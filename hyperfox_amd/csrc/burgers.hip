@@ -119,8 +119,9 @@ struct BLay {
 // two waves per SIMD, and small cells wait on each other's barriers.  When
 // three or more workgroups fit a CU's 160 KB of LDS the target is four
 // (128 VGPRs, a few spills in the set-up phases): measured on gfx950 for
-// 32,768 2-D p=3 cells, Burgers 4.9 -> 3.6 ms, nGamma 3.4 -> 3.1 ms (a target
-// of three ran nGamma at 3.8 ms).  Larger cells keep their LDS-bound count.
+// 32,768 2-D p=3 cells, before the phases were reworked, Burgers 4.9 -> 3.6 ms,
+// nGamma 3.4 -> 3.1 ms (a target of three ran nGamma at 3.8 ms); 1.91 and
+// 2.12 ms now.  Larger cells keep their LDS-bound count.
 template <int D, int P, int MDL>
 constexpr int burgers_waves() {
   constexpr long bytes = (long)BLay<D, P, MDL>::TOTAL * 8 + 1024;
@@ -128,7 +129,7 @@ constexpr int burgers_waves() {
   return w >= 3 ? 4 : (w < 1 ? 1 : (int)w);
 }
 
-// Cells whose working set does not fit the LDS (3-D p = 3: 279 KB) keep it
+// Cells whose working set does not fit the LDS (3-D p = 3: 341 KB) keep it
 // in a device workspace, one slab per workgroup in the same layout; the
 // workgroup barriers order those accesses as they order the LDS ones.
 template <int D, int P, int MDL>
@@ -146,7 +147,10 @@ constexpr bool burgers_in_workspace() {
 // device holds at once, so that the tables are read once per workgroup.
 // Measured, 18,432 2-D p=3 Burgers cells: 2.09 ms before, 1.08 ms (1.66 ms with
 // the shorter elimination alone).  Recomputing the index arithmetic for every
-// cell instead of keeping it in registers (no spills) took 1.26 ms.
+// cell instead of keeping it in registers (no spills) took 1.26 ms.  In 3-D a
+// whole assembly went 0.84 -> 0.56 ms (10,368 p=1 cells), 5.3 -> 2.9 ms (6,000
+// p=2) and 35.4 -> 14.8 ms (3,072 p=3, from the workspace), with 24, 108 and
+// 341 KB a cell where 18, 84 and 273 were.
 template <int D, int P, int MDL>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(burgers_waves<D, P, MDL>())))
 void burgers_cell_kernel(BurgersArgs a) {

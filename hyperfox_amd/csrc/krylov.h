@@ -60,9 +60,9 @@ struct KrylovOpts {
   int restart = 30;
   // BiCGStab: run the steady iterations between two residual checks as one
   // captured HIP graph (the same kernels in the same order, so the same
-  // results), when a preconditioner is given.  Off by default: measured no
-  // faster on gfx950 (the launches are already asynchronous), and each solve
-  // pays the capture
+  // results), when a preconditioner is given.  Off by default: measured at
+  // most 6 % faster on gfx950 (the launches are already asynchronous), and
+  // short solves are slower, as each pays the capture
   bool graph = false;
 };
 

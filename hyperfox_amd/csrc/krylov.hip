@@ -899,8 +899,13 @@ void KrylovWs::wait(int seq, hipStream_t s) const {
 constexpr int INLINE_PARTIALS = 2048;
 
 // Steps whose vectors span at most this many 256-row blocks leave the partials
-// of V^T w for every block of the next kernel to add up (k x 128 values out of
-// L2, about the time of the extra launch); longer ones reduce them first.
+// of V^T w for every block of the next kernel to add up; longer ones reduce
+// them first, one launch more per sum.  126 steps at restart 30, added up in
+// place / reduced first: one block 2.8 / 3.5 ms, 4 blocks 3.4 / 3.6, 10 to 60
+// level (3.7 to 3.9), 104 blocks 4.7 / 4.1, 127 blocks 4.3 / 3.8, 217 blocks
+// 5.8 / 4.2.  Reducing first wins from 65 on already (a second value per lane);
+// the line stays because it decides the order of the sums, and so the iterates,
+// of systems of 65 to 128 blocks.
 constexpr int GM_INLINE = 128;
 
 void fgmres(const BsrDev& A, const double* b, double* x, const PcApply& M, const KrylovOpts& o, KrylovInfo& info,

@@ -318,7 +318,7 @@ class HDGProblem:
 
     def set_solver_graphs(self, on):
         """BiCGStab steady iterations as one captured HIP graph (default off:
-        no faster on MI355X)."""
+        at best 6 % faster on MI355X, slower on short solves)."""
         check(lib.hfx_hdg_set_solver_graphs(self._h, 1 if on else 0))
 
     def set_krylov(self, method):

@@ -272,9 +272,9 @@ enum { HFX_KRYLOV_FGMRES = 0, HFX_KRYLOV_BICGSTAB = 1 };
 int hfx_hdg_set_krylov(hfx_hdg* h, int method);
 /* BiCGStab with a preconditioner runs the steady iterations between two
  * residual checks (8) as one captured HIP graph (on = 1) or as separate
- * launches (on = 0, the default: graphs measured no faster on MI355X, and
- * each solve pays the capture); the kernels and their order are the same, so
- * are the results.  No counterpart in the reference. */
+ * launches (on = 0, the default: on MI355X graphs measured at most 6 % faster,
+ * and short solves slower, as each pays the capture); the kernels and their
+ * order are the same, so are the results.  No counterpart in the reference. */
 int hfx_hdg_set_solver_graphs(hfx_hdg* h, int on);
 
 /* Trace solve (LinAlgebraInterface::solve, HDGSolver.cpp:699-708): FP64

@@ -21,7 +21,7 @@ from test_burgers_oracle import cole_hopf, regression_case  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
-# 3-D p = 3: the cell's working set (279 KB) is kept in a device workspace
+# 3-D p = 3: the cell's working set (341 KB) is kept in a device workspace
 CASES = [(2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (3, 1), (3, 2), (3, 3)]
 
 

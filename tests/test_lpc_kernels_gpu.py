@@ -1,5 +1,5 @@
 """The FP32 products of the learned preconditioner at every block size (the inputs of the encoders and decoders are
-b^2 and b^2 + 1 wide, so their 16-wide chunks are ragged or unaligned) and at row counts around the 128-row tiles and
+b^2 and b^2 + 1 wide, so their 16-wide chunks are ragged or unaligned) and at row counts around the 64-row tiles and
 the parts of the weight gradient: outputs, loss and gradient against the FP64 oracle.
 
 Bound of the gradient: FP32 sums of up to a few thousand terms through eight layers; 2e-4 of each tensor's norm is

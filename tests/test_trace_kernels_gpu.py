@@ -79,8 +79,8 @@ def test_reconstruction(dim, p, n):
 @pytest.mark.parametrize('restart', [1, 2, 8, 9, 17, 33, 63])
 @pytest.mark.parametrize('n', [1, 7, 19])
 def test_gmres_against_a_dense_solve(n, restart):
-    """Restart lengths around the register tiles (8, 16 and 32 columns), one and several row blocks, an iteration budget
-    inside a cycle, and convergence inside a cycle.  At rtol the residual is at most rtol ||b||, so the error is at
+    """Restart lengths below and above the 4 to 15 steps that these systems need (longer cycles are in the tests below),
+    one and several row blocks, an iteration budget inside a cycle, and convergence inside a cycle.  At rtol the residual is at most rtol ||b||, so the error is at
     most cond(A) rtol ||x||."""
     print('gmres', n, restart, flush=True)
     rng = np.random.default_rng(n)
