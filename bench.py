@@ -201,22 +201,23 @@ PC_NAMES = {'jacobi': 1, 'block-jacobi': 2, 'learned': 3, 'ilu0': 4, 'ilu0-natur
 
 
 def solver_bytes_per_iter(n, nb, bs, nnzb, method, pc='block-jacobi'):
-    """Algorithmic HBM bytes of one Krylov iteration: BiCGStab = 2 BSR SpMV
-    (values, column ids, x and y once) + 2 preconditioner applies + 21 vector
-    passes; FGMRES at Krylov dimension ~15 = 1 SpMV + 1 apply + 2 x (2k + 3)
-    vector passes (two Gram-Schmidt sweeps).  Applies: point Jacobi 3 vector
-    passes; block Jacobi the inverse diagonal blocks + 2 passes; ILU(0) every
+    """HBM bytes of one Krylov iteration as the kernels run it: BiCGStab = 2 BSR
+    SpMV (values, column ids, x and y once) + 2 preconditioner applies + 17
+    vector passes; FGMRES(30), mean over a cycle (15.5 basis rows) = 1 SpMV + 1
+    apply + 56 vector passes (the basis read three times, rows past the 16th a
+    fourth time, and 6 passes).  Applies: point and block Jacobi, fused into the
+    vector kernel before them, the inverse diagonal + 1 pass; ILU(0) every
     factor block (FP64) with its column id + the inverse pivot blocks + 4
     passes (ilu0-f32: the factor blocks in FP32); learned the FP32 BSR matrix
     + column ids + 2 passes."""
     spmv = nnzb * bs * bs * 8 + nnzb * 4 + 2 * n * 8
-    apply = {'jacobi': 3 * n * 8, 'block-jacobi': nb * bs * bs * 8 + 2 * n * 8,
+    apply = {'jacobi': 2 * n * 8, 'block-jacobi': nb * bs * bs * 8 + n * 8,
              'ilu0': nnzb * bs * bs * 8 + nnzb * 8 + nb * bs * bs * 8 + 4 * n * 8,
              'ilu0-f32': nnzb * bs * bs * 4 + nnzb * 8 + nb * bs * bs * 4 + 4 * n * 8,
              'learned': nnzb * bs * bs * 4 + nnzb * 4 + 2 * n * 8}[pc.replace('-natural', '')]
     if method == 'bicgstab':
-        return 2 * spmv + 2 * apply + 21 * n * 8
-    return spmv + apply + 2 * (2 * 15 + 3) * n * 8
+        return 2 * spmv + 2 * apply + 17 * n * 8
+    return spmv + apply + 56 * n * 8
 
 
 def timed_solve(hf, prob, method, pc, maxits, warm=True):
